@@ -1934,16 +1934,27 @@ __device__ __forceinline__ TileRec rec_tile_at(const int4* __restrict__ r, int t
 // (src/AMGSolver.cu:1257-1277), in one workgroup of 1024 threads, for a level 0 of one
 // tile without neighbours (the root) whose 8 children are the whole of level 1.  Level 1
 // is then a dense 16^3 block: its x (masked to INTERIOR cells, with a zero halo at the
-// domain boundary) and face coefficients stay in LDS for every pass, so a pass costs LDS
-// reads and a barrier instead of a launch and a memory round trip.  Group g (128 threads,
-// 4 cells each) holds the level-1 tile of octant g.  Every step does the arithmetic of
-// the per-pass kernel it replaces (gs_color, jacobi, residual_restrict, fas_save,
-// fas_prolong_v, jacobi's r.z partial and prolongation into level 2), so the results
-// are bit-identical; the root's steps (FAS save, coarsest iterations) are the per-tile
-// functions themselves, on 512 threads (the other 512 redo them without writing).
-// phase 1: pre-smoothing, residual + restriction, the root's FAS save; phase 2: the
-// prolongation to level 1 and its post-smoothing; phase 3: both with the coarsest
-// iterations (mu times) in between.
+// domain boundary) stays in LDS for every pass, its face coefficients in registers, so a
+// pass costs the LDS reads of x and a barrier instead of a launch and a memory round trip.
+// Group g (128 threads, 4 cells each) holds the level-1 tile of octant g; the root's x and
+// right-hand side stay in LDS too, and its 512 cells are two a thread, one of each colour,
+// on the first 256 threads.  Every step does the arithmetic of the per-pass kernel it
+// replaces (gs_color, jacobi, residual_restrict, fas_save, coarsest_tile, fas_prolong_v,
+// jacobi's r.z partial), so the results are bit-identical.
+// phase 1: level 1's FAS save, pre-smoothing, residual + restriction, the root's FAS save;
+// phase 2: the prolongation to level 1, its post-smoothing and the prolongation into level
+// 2; phase 3: both with the coarsest iterations (mu times) in between.
+//
+// One CU does all of it, so a pass is bound by instruction issue (16 waves on 4 SIMDs) and
+// the chain LDS read - seven dependent fmas - division - LDS write - barrier.  Hence: a
+// thread's cells are kept colour by colour (only a colour's own cells are computed in its
+// pass, with no selects), the + face coefficients are registers, a division is a product
+// with the FP64 reciprocal of the diagonal, and the root's passes run on one wave per SIMD
+// with no memory traffic between them.  (MI355X, W-cycle settings with 10 coarsest
+// iterations and mu = 2, i.e. 8 passes on level 1 and 40 on the root: 19.6 us a visit, 0.17 us
+// a root pass; 44.2 us with every cell computed in every pass and the root's steps staged
+// through memory and computed twice, and another 9 us for level 1's FAS save and the
+// prolongation into level 2 in launches of their own.)
 struct BottomArgs {
     const int4* rec0;    // the root's record
     int root;            // the root tile
@@ -1965,32 +1976,49 @@ struct BottomArgs {
 template <bool Q>
 struct BottomLds {
     float x[18 * 18 * 18];                                    // level 1, masked, zero halo
-    std::conditional_t<Q, uint16_t, float> c[3][4096];        // negative-face coefficients
-    float res[4096];                                          // residuals for the restriction
-    Lds<float, Q> root[2];                                    // the root's steps, two copies
+    union {
+        std::conditional_t<Q, uint16_t, float> c[3][4096];    // negative-face coefficients, while they are read in
+        float res[4096];                                      // residuals for the restriction
+    };
+    float rx[1000];                                           // the root's x, masked, zero halo
+    float rb[512];                                            // its right-hand side
     double red[16];
 };
 
 __device__ __forceinline__ int bx(int i, int j, int k) { return (i + 1) * 324 + (j + 1) * 18 + (k + 1); }
 __device__ __forceinline__ int bc(int i, int j, int k) { return (i << 8) | (j << 4) | k; }
 
-template <bool Q>
-__device__ __forceinline__ float bottom_lap(const BottomLds<Q>& s, int i, int j, int k, float x0, const float c[3], float d,
-                                            float h)
+// n / d for the FP64 reciprocal rd = 1 / d: the correctly rounded FP32 quotient.  The product
+// is within 2^-52 of n / d, and no quotient of two FP32 numbers lies within 2^-49 of the
+// midpoint of two neighbouring normal FP32 numbers.
+__device__ __forceinline__ float quotient(float n, double rd) { return float(double(n) * rd); }
+
+// one cell of a block kept in LDS: A x at LDS index c (strides si, sj, 1) with the face
+// coefficients in registers (neg_lap's order)
+__device__ __forceinline__ float block_lap(const float* x, int c, int si, int sj, float x0, const float (&cm)[3],
+                                           const float (&cp)[3], float d)
 {
-    if (d == 0) return 0.0f;
-    // the + face coefficient is the + neighbour's own; h where the level ends (its x is 0 there)
-    const float cp0 = i < 15 ? lds_coef(s.c[0][bc(i + 1, j, k)], h) : h;
-    const float cp1 = j < 15 ? lds_coef(s.c[1][bc(i, j + 1, k)], h) : h;
-    const float cp2 = k < 15 ? lds_coef(s.c[2][bc(i, j, k + 1)], h) : h;
+    const float v0 = x[c - si], v1 = x[c + si], v2 = x[c - sj], v3 = x[c + sj], v4 = x[c - 1], v5 = x[c + 1];
     float r = x0 * d;
-    r = fmaf(c[0], s.x[bx(i - 1, j, k)], r);
-    r = fmaf(cp0, s.x[bx(i + 1, j, k)], r);
-    r = fmaf(c[1], s.x[bx(i, j - 1, k)], r);
-    r = fmaf(cp1, s.x[bx(i, j + 1, k)], r);
-    r = fmaf(c[2], s.x[bx(i, j, k - 1)], r);
-    r = fmaf(cp2, s.x[bx(i, j, k + 1)], r);
-    return r;
+    r = fmaf(cm[0], v0, r);
+    r = fmaf(cp[0], v1, r);
+    r = fmaf(cm[1], v2, r);
+    r = fmaf(cp[1], v3, r);
+    r = fmaf(cm[2], v4, r);
+    r = fmaf(cp[2], v5, r);
+    return d == 0 ? 0.0f : r;
+}
+
+// four consecutive cells, pairs swapped when odd: [2s] is then the pair's red cell, [2s + 1] its black one
+template <typename E>
+__device__ __forceinline__ void by_colour(E (&v)[4], bool odd)
+{
+#pragma unroll
+    for (int s = 0; s < 4; s += 2) {
+        const E a = v[s], b = v[s + 1];
+        v[s] = odd ? b : a;
+        v[s + 1] = odd ? a : b;
+    }
 }
 
 template <bool Q>
@@ -2000,7 +2028,6 @@ __global__ __launch_bounds__(1024) void cycle_bottom(TopoView tp, BottomArgs a, 
     if (S[S_DONE] != 0.0) return;   // the solve has stopped (uniform)
     // the group is uniform over a wave (two waves a group)
     const int g = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 7)), tid = threadIdx.x & 127;
-    const int4* r0p = a.rec0;
     const int root = a.root;
     const int t = a.tile[g];   // the level-1 tile of octant g (kernel arguments: no dependent load)
     const int tmeta = a.type[g];
@@ -2008,14 +2035,27 @@ __global__ __launch_bounds__(1024) void cycle_bottom(TopoView tp, BottomArgs a, 
     const size_t v0 = size_t(t) * 512 + 4 * tid;
     const int li = tid >> 4, lj = (tid >> 1) & 7, lk0 = 4 * (tid & 1);   // the thread's cells in the tile
     const int gi = 8 * (g & 1) + li, gj = 8 * ((g >> 1) & 1) + lj, gk0 = 8 * ((g >> 2) & 1) + lk0;
-    float x[4], b[4], cf[4][3], d[4];
+    const bool odd = (li + lj) & 1;
+    // slot 2s + col holds the pair's cell of colour col, at k = gk0 + 2s + (odd ^ col)
+    auto slot_k = [&](int c) { return gk0 + (c & 2) + (int(odd) ^ (c & 1)); };
+    float x[4], b[4], cm[4][3], cp[4][3], d[4];
+    double rd[4];
     uint8_t ct[4];
+    // ---- the root's cells of this thread (threads 0..255): a pair along k, [0] red, [1] black
+    const bool rootw = threadIdx.x < 256;
+    const int ri = int(threadIdx.x >> 5) & 7, rj = (threadIdx.x >> 2) & 7, rk0 = 2 * (threadIdx.x & 3);
+    const bool rodd = (ri + rj) & 1;
+    const float h0 = tp.h0;
+    float rcm[2][3], rcp[2][3], rdg[2], rx0[2];
+    double rrd[2];
+    uint8_t rct[2];
     // ---- level 1 into registers and LDS
     {
-        float xr[4];
+        float xr[4], cf[4][3], dd[4];
         vload<4>(a.X + v0, xr);
         vload<4>(a.B + v0, b);
         vload<4>(tp.ctype + v0, ct);
+        const bool dv = !Q && tp.derive && (tmeta & LEAF);
         if constexpr (Q) {
             uint16_t q[4][4];
 #pragma unroll
@@ -2027,11 +2067,10 @@ __global__ __launch_bounds__(1024) void cycle_bottom(TopoView tp, BottomArgs a, 
                     cf[c][e] = float(__builtin_bit_cast(_Float16, q[e][c])) * h;
                     s.c[e][bc(gi, gj, gk0 + c)] = q[e][c];
                 }
-                d[c] = float(__builtin_bit_cast(_Float16, q[3][c])) * h;
+                dd[c] = float(__builtin_bit_cast(_Float16, q[3][c])) * h;
             }
         } else {
             float q[4][4];
-            const bool dv = tp.derive && (tmeta & LEAF);
 #pragma unroll
             for (int e = 0; e < 3; ++e) vload<4>(a.C.c[e] + v0, q[e]);
             if (!dv) vload<4>(a.C.c[3] + v0, q[3]);
@@ -2042,7 +2081,30 @@ __global__ __launch_bounds__(1024) void cycle_bottom(TopoView tp, BottomArgs a, 
                     cf[c][e] = q[e][c];
                     s.c[e][bc(gi, gj, gk0 + c)] = q[e][c];
                 }
-                d[c] = dv ? 0.0f : q[3][c];
+                dd[c] = dv ? 0.0f : q[3][c];
+            }
+        }
+        // the root: types, coefficients and (cells that its FAS save leaves alone) the saved x
+        if (rootw) {
+            const size_t rv = size_t(root) * 512;
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                const int rk = rk0 + (int(rodd) ^ e), v = cidx(ri, rj, rk);
+                rct[e] = tp.ctype[rv + v];
+                rx0[e] = a.X0[rv + v];
+                const int nv[3] = {ri < 7 ? v + 64 : -1, rj < 7 ? v + 8 : -1, rk < 7 ? v + 1 : -1};
+#pragma unroll
+                for (int ax = 0; ax < 3; ++ax) {
+                    if constexpr (Q) {
+                        rcm[e][ax] = coef_q(a.C.q[ax], rv + v, h0);
+                        rcp[e][ax] = nv[ax] < 0 ? h0 : coef_q(a.C.q[ax], rv + nv[ax], h0);
+                    } else {
+                        rcm[e][ax] = a.C.c[ax][rv + v];
+                        rcp[e][ax] = nv[ax] < 0 ? h0 : a.C.c[ax][rv + nv[ax]];
+                    }
+                }
+                if constexpr (Q) rdg[e] = coef_q(a.C.q[3], rv + v, h0);
+                else rdg[e] = a.C.c[3][rv + v];
             }
         }
 #pragma unroll
@@ -2050,92 +2112,150 @@ __global__ __launch_bounds__(1024) void cycle_bottom(TopoView tp, BottomArgs a, 
             x[c] = ct[c] == INTERIOR ? xr[c] : 0.0f;
             s.x[bx(gi, gj, gk0 + c)] = x[c];
         }
-        // the zero halo of the 16^3 block
+        // the zero halos of the 16^3 block and of the root
         for (int m = threadIdx.x; m < 18 * 18 * 18; m += 1024) {
             const int hi = m / 324, hj = (m / 18) % 18, hk = m % 18;
             if (hi == 0 || hi == 17 || hj == 0 || hj == 17 || hk == 0 || hk == 17) s.x[m] = 0.0f;
         }
+        if (threadIdx.x < 1000) s.rx[threadIdx.x] = 0.0f;
         __syncthreads();
-        if constexpr (!Q) {
-            if (tp.derive && (tmeta & LEAF)) {
-                // derived_diag: d = 0 - c-(x) - c+(x) - ..., c+ = -h where the level ends
 #pragma unroll
-                for (int c = 0; c < 4; ++c) {
-                    const int k = gk0 + c;
-                    const float cp0 = gi < 15 ? s.c[0][bc(gi + 1, gj, k)] : -h;
-                    const float cp1 = gj < 15 ? s.c[1][bc(gi, gj + 1, k)] : -h;
-                    const float cp2 = k < 15 ? s.c[2][bc(gi, gj, k + 1)] : -h;
-                    float dd = 0.0f;
-                    dd = dd - cf[c][0];
-                    dd = dd - cp0;
-                    dd = dd - cf[c][1];
-                    dd = dd - cp1;
-                    dd = dd - cf[c][2];
-                    dd = dd - cp2;
-                    d[c] = (ct[c] & INTERIOR) ? dd : 0.0f;
-                }
+        for (int c = 0; c < 4; ++c) {
+            const int k = gk0 + c;
+            // the + face coefficient is the + neighbour's own; h where the level ends (its x is 0 there)
+            const float c0 = gi < 15 ? lds_coef(s.c[0][bc(gi + 1, gj, k)], h) : h;
+            const float c1 = gj < 15 ? lds_coef(s.c[1][bc(gi, gj + 1, k)], h) : h;
+            const float c2 = k < 15 ? lds_coef(s.c[2][bc(gi, gj, k + 1)], h) : h;
+            cp[c][0] = c0;
+            cp[c][1] = c1;
+            cp[c][2] = c2;
+            if (dv) {
+                // derived_diag: d = 0 - c-(x) - c+(x) - ..., c+ = -h where the level ends
+                float v = 0.0f;
+                v = v - cf[c][0];
+                v = v - (gi < 15 ? c0 : -h);
+                v = v - cf[c][1];
+                v = v - (gj < 15 ? c1 : -h);
+                v = v - cf[c][2];
+                v = v - (k < 15 ? c2 : -h);
+                dd[c] = (ct[c] & INTERIOR) ? v : 0.0f;
             }
+            d[c] = dd[c];
+#pragma unroll
+            for (int e = 0; e < 3; ++e) cm[c][e] = cf[c][e];
+        }
+        by_colour(x, odd);
+        by_colour(b, odd);
+        by_colour(ct, odd);
+        by_colour(d, odd);
+#pragma unroll
+        for (int e = 0; e < 3; ++e) {
+            float m4[4] = {cm[0][e], cm[1][e], cm[2][e], cm[3][e]}, p4[4] = {cp[0][e], cp[1][e], cp[2][e], cp[3][e]};
+            by_colour(m4, odd);
+            by_colour(p4, odd);
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                cm[c][e] = m4[c];
+                cp[c][e] = p4[c];
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < 4; ++c) rd[c] = 1.0 / double(d[c]);
+        if (rootw) {
+#pragma unroll
+            for (int e = 0; e < 2; ++e) rrd[e] = 1.0 / double(rdg[e]);
         }
     }
     const int n = a.iters;
-    // one smoothing pass on level 1: colour `col` of red-black SOR (col >= 0) or a damped-Jacobi
-    // sweep (col < 0, `save`: with the FAS save of NONLEAF tiles; `dot`: returns sum b x_out)
-    auto pass = [&](int col, bool save, bool dot, float* xo) -> double {
-        double acc = 0;
-        float ax[4];
+    int lx[4];   // the cells' places in s.x
 #pragma unroll
-        for (int c = 0; c < 4; ++c) ax[c] = bottom_lap(s, gi, gj, gk0 + c, x[c], cf[c], d[c], h);
-        if (col >= 0) {
+    for (int c = 0; c < 4; ++c) lx[c] = bx(gi, gj, slot_k(c));
+    auto lap = [&](int c) { return block_lap(s.x, lx[c], 324, 18, x[c], cm[c], cp[c], d[c]); };
+    // four cells in the order of their places, to or from memory
+    auto put4 = [&](float* p, const float (&v)[4]) {
+        float o[4] = {v[0], v[1], v[2], v[3]};
+        by_colour(o, odd);
+        vstore<4>(p, o);
+    };
+    // one colour of red-black SOR
+    auto colour_pass = [&](auto colour) {
+        constexpr int col = decltype(colour)::value;
 #pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                if (((li + lj + lk0 + c) & 1) != col) continue;
-                const float delta = (ct[c] & INTERIOR) ? (b[c] - ax[c]) / d[c] : 0.0f;
-                x[c] = float(double(x[c]) + double(delta) * a.omega);
-                s.x[bx(gi, gj, gk0 + c)] = x[c];   // 0 on other cells already
-            }
-            __syncthreads();
-            return 0;
+        for (int q = 0; q < 2; ++q) {
+            const int c = 2 * q + col;
+            const float ax = lap(c);
+            const float delta = (ct[c] & INTERIOR) ? quotient(b[c] - ax, rd[c]) : 0.0f;
+            x[c] = float(double(x[c]) + double(delta) * a.omega);
+            s.x[lx[c]] = x[c];   // 0 on other cells already
         }
-        const bool sv = save && (tmeta & NONLEAF);
+        __syncthreads();
+    };
+    using Red = std::integral_constant<int, 0>;
+    using Black = std::integral_constant<int, 1>;
+    // the FAS save of NONLEAF tiles (fas_save): b += A x, the x saved
+    auto fas_save1 = [&]() {
+        if (!(tmeta & NONLEAF)) return;
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-            if (sv) {
-                if (ct[c] & INTERIOR) {
-                    b[c] = b[c] + ax[c];
-                    a.X0[v0 + c] = x[c];
-                } else {
-                    b[c] = 0.0f;
-                }
-            }
-            const float delta = (ct[c] & INTERIOR) ? (b[c] - ax[c]) / d[c] : 0.0f;
-            xo[c] = x[c] + a.w * delta;
-            if (dot && (tmeta & LEAF)) acc += double(b[c]) * double(xo[c]);
+            const bool in = ct[c] & INTERIOR;
+            b[c] = in ? b[c] + lap(c) : 0.0f;
+            if (in) a.X0[v0 + (slot_k(c) - gk0)] = x[c];
         }
-        if (sv) vstore<4>(a.B + v0, b);
+        put4(a.B + v0, b);
+    };
+    float xo[4];
+    // a damped-Jacobi sweep (`save`: with the FAS save; `dot`: returns sum b x_out in the cells' order)
+    auto sweep = [&](bool save, bool dot) -> double {
+        double acc = 0;
+        if (save) fas_save1();
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const float delta = (ct[c] & INTERIOR) ? quotient(b[c] - lap(c), rd[c]) : 0.0f;
+            xo[c] = x[c] + a.w * delta;
+        }
+        if (dot && (tmeta & LEAF)) {
+            float bo[4] = {b[0], b[1], b[2], b[3]}, xn[4] = {xo[0], xo[1], xo[2], xo[3]};
+            by_colour(bo, odd);
+            by_colour(xn, odd);
+#pragma unroll
+            for (int c = 0; c < 4; ++c) acc += double(bo[c]) * double(xn[c]);
+        }
         __syncthreads();   // every read of this sweep is done before x changes
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
             x[c] = ct[c] == INTERIOR ? xo[c] : 0.0f;
-            s.x[bx(gi, gj, gk0 + c)] = x[c];
+            s.x[lx[c]] = x[c];
         }
         __syncthreads();
         return acc;
     };
-    float xo[4];
+    // the root: x of a cell and A x
+    const int rl[2] = {SX(ri, rj, rk0 + int(rodd)), SX(ri, rj, rk0 + 1 - int(rodd))};
+    const int rv[2] = {cidx(ri, rj, rk0 + int(rodd)), cidx(ri, rj, rk0 + 1 - int(rodd))};
+    float rxv[2] = {0.0f, 0.0f}, rbv[2] = {0.0f, 0.0f};
+    auto root_lap = [&](int e) { return block_lap(s.rx, rl[e], 100, 10, rxv[e], rcm[e], rcp[e], rdg[e]); };
     if (a.phase & 1) {
         // pre-smoothing (order 0)
-        for (int it = 0; it < n; ++it) {
-            if (a.rbgs) {
-                pass(0, false, false, xo);
-                pass(1, false, false, xo);
-            } else {
-                pass(-1, a.fas_save1 && it == 0, false, xo);
+        if (a.rbgs) {
+            if (a.fas_save1) {
+                fas_save1();
+                __syncthreads();   // every read of x for the save is done before x changes
             }
+            for (int it = 0; it < n; ++it) {
+                colour_pass(Red{});
+                colour_pass(Black{});
+            }
+        } else {
+            for (int it = 0; it < n; ++it) sweep(a.fas_save1 && it == 0, false);
         }
         // residual and restriction into the root (residual_restrict)
+        __syncthreads();   // (res takes the place of the coefficients)
+        {
+            float rv4[4];
 #pragma unroll
-        for (int c = 0; c < 4; ++c)
-            s.res[g * 512 + 4 * tid + c] = b[c] - bottom_lap(s, gi, gj, gk0 + c, x[c], cf[c], d[c], h);
+            for (int c = 0; c < 4; ++c) rv4[c] = b[c] - lap(c);
+            put4(&s.res[g * 512 + 4 * tid], rv4);
+        }
         __syncthreads();
         if (tid < 64) {
             const int fl0 = tid / 16 * 2, fl1 = (tid / 4) % 4 * 2, fl2 = tid % 4 * 2;
@@ -2149,45 +2269,130 @@ __global__ __launch_bounds__(1024) void cycle_bottom(TopoView tp, BottomArgs a, 
                         rs += s.res[g * 512 + cidx(fl0 + ii, fl1 + jj, fl2 + kk)];
                         xs += s.x[bx(8 * (g & 1) + fl0 + ii, 8 * ((g >> 1) & 1) + fl1 + jj, 8 * ((g >> 2) & 1) + fl2 + kk)];
                     }
-            const size_t pidx = size_t(root) * 512 + cidx(4 * (g & 1) + (fl0 >> 1), 4 * ((g >> 1) & 1) + (fl1 >> 1),
-                                                         4 * ((g >> 2) & 1) + (fl2 >> 1));
-            a.B[pidx] = rs * a.Rr;
-            a.X[pidx] = xs / 8;
+            const int p0 = 4 * (g & 1) + (fl0 >> 1), p1 = 4 * ((g >> 1) & 1) + (fl1 >> 1), p2 = 4 * ((g >> 2) & 1) + (fl2 >> 1);
+            s.rb[cidx(p0, p1, p2)] = rs * a.Rr;
+            s.rx[SX(p0, p1, p2)] = xs / 8;
         }
         // level 1's x after the pre-smoothing (read back by phase 2 when the coarsest solve
         // runs in between; the jacobi ping-pong buffer is not written)
-        vstore<4>(a.X + v0, x);
+        if (a.phase == 1) put4(a.X + v0, x);
         __syncthreads();
-        if (a.nonleaf0) {
-            TileRec r = rec_tile_at(r0p, int(threadIdx.x & 511));
-            fas_save_tile<512, Q>(tp, r, s.root[threadIdx.x >> 9], a.X, a.C, a.B, a.X0, threadIdx.x < 512);
-            __syncthreads();
+        if (rootw) {
+            const size_t rbase = size_t(root) * 512;
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                const float xs = s.rx[rl[e]];
+                a.X[rbase + rv[e]] = xs;   // as the restriction leaves it (the passes below write INTERIOR cells)
+                rxv[e] = rct[e] == INTERIOR ? xs : 0.0f;
+                rbv[e] = s.rb[rv[e]];
+                s.rx[rl[e]] = rxv[e];
+            }
         }
+        __syncthreads();
+        if (a.nonleaf0 && rootw) {
+            // the root's FAS save
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                const bool in = rct[e] & INTERIOR;
+                rbv[e] = in ? rbv[e] + root_lap(e) : 0.0f;
+                if (in) rx0[e] = rxv[e];
+            }
+        }
+        if (rootw) {
+            const size_t rbase = size_t(root) * 512;
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                a.B[rbase + rv[e]] = rbv[e];
+                a.X0[rbase + rv[e]] = rx0[e];
+            }
+        }
+        __syncthreads();
     }
     if (a.phase == 3) {
+        // the coarsest iterations on the root (coarsest_tile)
+        auto root_pass = [&](auto colour) {
+            constexpr int e = decltype(colour)::value;
+            if (rootw) {
+                const float ax = root_lap(e);
+                const float delta = (rct[e] & INTERIOR) ? quotient(rbv[e] - ax, rrd[e]) : 0.0f;
+                const float xn = float(double(rxv[e]) + double(delta) * a.omega);
+                rxv[e] = rct[e] == INTERIOR ? xn : 0.0f;
+                s.rx[rl[e]] = rxv[e];
+            }
+            __syncthreads();
+        };
         const int it1 = a.rbgs ? a.coarsest_iters / 2 : a.coarsest_iters;
         for (int i = 0; i < a.mu; ++i) {
-            TileRec r = rec_tile_at(r0p, int(threadIdx.x & 511));
-            coarsest_tile<512, Q>(tp, r, s.root[threadIdx.x >> 9], a.X, a.C, a.B, a.rbgs, it1, a.rbgs ? it1 : 0, 0,
-                                  a.omega, a.w, threadIdx.x < 512);
-            __syncthreads();
+            if (a.rbgs) {
+                for (int it = 0; it < it1; ++it) {
+                    root_pass(Red{});
+                    root_pass(Black{});
+                }
+                for (int it = 0; it < it1; ++it) {
+                    root_pass(Black{});
+                    root_pass(Red{});
+                }
+            } else {
+                for (int it = 0; it < it1; ++it) {
+                    float xn[2];
+                    if (rootw) {
+#pragma unroll
+                        for (int e = 0; e < 2; ++e) {
+                            const float delta = (rct[e] & INTERIOR) ? quotient(rbv[e] - root_lap(e), rrd[e]) : 0.0f;
+                            xn[e] = rxv[e] + a.w * delta;
+                        }
+                    }
+                    __syncthreads();   // every read of this sweep is done before x changes
+                    if (rootw) {
+#pragma unroll
+                        for (int e = 0; e < 2; ++e) {
+                            rxv[e] = rct[e] == INTERIOR ? xn[e] : 0.0f;
+                            s.rx[rl[e]] = rxv[e];
+                        }
+                    }
+                    __syncthreads();
+                }
+            }
+        }
+        if (rootw && it1 > 0 && a.mu > 0) {
+            const size_t rbase = size_t(root) * 512;
+#pragma unroll
+            for (int e = 0; e < 2; ++e) a.X[rbase + rv[e]] = rxv[e];
         }
     }
     if (a.phase & 2) {
         // the prolongation to level 1 (fas_prolong_v; no GHOST tile on a complete level 1)
-        {
+        float cx[2], cx0[2];
+        if (a.phase == 2) {
             const size_t pb = size_t(root) * 512 + cidx(gi >> 1, gj >> 1, gk0 >> 1);
             const float2 xc = *reinterpret_cast<const float2*>(a.X + pb), x0c = *reinterpret_cast<const float2*>(a.X0 + pb);
-            const float cx[2] = {xc.x, xc.y}, cx0[2] = {x0c.x, x0c.y};
+            cx[0] = xc.x; cx[1] = xc.y;
+            cx0[0] = x0c.x; cx0[1] = x0c.y;
+        } else {
+            // through LDS: x is there (with no coarsest iteration it is the restriction's, unmasked), X0 takes rb's place
+            const bool ran = a.mu > 0 && (a.rbgs ? a.coarsest_iters / 2 : a.coarsest_iters) > 0;
+            if (rootw) {
 #pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                x[c] = (ct[c] & INTERIOR) ? x[c] + a.P * (cx[c >> 1] - cx0[c >> 1]) : 0.0f;
-                s.x[bx(gi, gj, gk0 + c)] = x[c];
+                for (int e = 0; e < 2; ++e) {
+                    s.rb[rv[e]] = rx0[e];
+                    if (!ran) s.rx[rl[e]] = a.X[size_t(root) * 512 + rv[e]];
+                }
             }
             __syncthreads();
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                cx[e] = s.rx[SX(gi >> 1, gj >> 1, (gk0 >> 1) + e)];
+                cx0[e] = s.rb[cidx(gi >> 1, gj >> 1, (gk0 >> 1) + e)];
+            }
         }
-        // post-smoothing (order 1); the last Jacobi sweep sums b.x = r.z and prolongs into level 2,
-        // whose x and types are loaded before that sweep
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            x[c] = (ct[c] & INTERIOR) ? x[c] + a.P * (cx[c >> 1] - cx0[c >> 1]) : 0.0f;
+            s.x[lx[c]] = x[c];
+        }
+        __syncthreads();
+        // post-smoothing (order 1); the last Jacobi sweep sums b.x = r.z.  The prolongation into
+        // level 2 follows; level 2's x and types are loaded before the last iteration
         const int oc = (li >> 2) | ((lj >> 2) << 1) | ((lk0 >> 2) << 2);
         const int ch = a.push ? a.child[8 * g + oc] : -1;
         float pxf[4][8];
@@ -2195,23 +2400,23 @@ __global__ __launch_bounds__(1024) void cycle_bottom(TopoView tp, BottomArgs a, 
         float px0[4];
         double acc = 0;
         for (int it = 0; it < n; ++it) {
-            if (a.rbgs) {
-                pass(1, false, false, xo);
-                pass(0, false, false, xo);
-            } else {
-                if (it == n - 1 && ch >= 0) {
-                    vload<4>(a.X0 + v0, px0);
+            if (it == n - 1 && ch >= 0) {
+                vload<4>(a.X0 + v0, px0);
 #pragma unroll
-                    for (int ab = 0; ab < 4; ++ab) {
-                        const size_t fb = size_t(ch) * 512 + cidx(2 * (li & 3) + (ab >> 1), 2 * (lj & 3) + (ab & 1), 0);
-                        vload<8>(a.X + fb, pxf[ab]);
-                        vload<8>(tp.ctype + fb, pcf[ab]);
-                    }
+                for (int ab = 0; ab < 4; ++ab) {
+                    const size_t fb = size_t(ch) * 512 + cidx(2 * (li & 3) + (ab >> 1), 2 * (lj & 3) + (ab & 1), 0);
+                    vload<8>(a.X + fb, pxf[ab]);
+                    vload<8>(tp.ctype + fb, pcf[ab]);
                 }
-                acc = pass(-1, false, a.rz && it == n - 1, xo);
+            }
+            if (a.rbgs) {
+                colour_pass(Black{});
+                colour_pass(Red{});
+            } else {
+                acc = sweep(false, a.rz && it == n - 1);
             }
         }
-        vstore<4>(a.X + v0, x);
+        put4(a.X + v0, x);
         if (a.rz) {
             // the tile's b.x partial, summed as block_sum sums a 128-thread workgroup's
             for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
@@ -2225,14 +2430,16 @@ __global__ __launch_bounds__(1024) void cycle_bottom(TopoView tp, BottomArgs a, 
             }
         }
         if (ch >= 0) {
-            // jacobi's prolongation into the children (level 2) from the last sweep's x
+            // the prolongation into the children (level 2) from the last pass's x
             const bool ghost = (a.ghost >> (8 * g + oc)) & 1ull;
+            float xc[4] = {x[0], x[1], x[2], x[3]};
+            by_colour(xc, odd);
 #pragma unroll
             for (int ab = 0; ab < 4; ++ab) {
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
                     const bool in = pcf[ab][e] & INTERIOR;
-                    const float c1 = xo[e >> 1], c0 = px0[e >> 1];
+                    const float c1 = xc[e >> 1], c0 = px0[e >> 1];
                     pxf[ab][e] = ghost ? (in ? c1 : 0.0f) : (in ? pxf[ab][e] + a.P * (c1 - c0) : 0.0f);
                 }
                 const size_t fb = size_t(ch) * 512 + cidx(2 * (li & 3) + (ab >> 1), 2 * (lj & 3) + (ab & 1), 0);
@@ -3231,7 +3438,7 @@ void launch_cycle_bottom(const DevGrid& d, int phase, float* X, float* X0, float
                          const double* S, hipStream_t st)
 {
     if (!cycle_bottom_available(d)) throw std::logic_error("cycle_bottom: levels 0 and 1 do not fit one workgroup");
-    if (push && (rbgs || iters < 1 || !jacobi_push_available(d, 1)))
+    if (push && (iters < 1 || !jacobi_push_available(d, 1)))
         throw std::invalid_argument("cycle_bottom: the prolongation to level 2 cannot ride on level 1's last sweep");
     if (rz && (rbgs || iters < 1)) throw std::invalid_argument("cycle_bottom: r.z partials come from a Jacobi sweep");
     k::BottomArgs a;

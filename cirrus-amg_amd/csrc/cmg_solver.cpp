@@ -920,6 +920,12 @@ int cycle_mu(const cmg_solve_opts* o)
     return o->cycle == CMG_CYCLE_FAS_V ? 1 : 2;
 }
 
+// this level of a cycle is the upper one of the two that one workgroup runs
+bool cycle_bottom_runs(const DevGrid& d, int level, bool x_zero)
+{
+    return level == 1 && level < d.max_level && !x_zero && cycle_bottom_available(d);
+}
+
 void coarsest(const CycleCtx& c)
 {
     DevGrid& d = c.s->g->dev;
@@ -952,14 +958,14 @@ bool cycle_step(const CycleCtx& c, int level, bool x_zero, bool fas_save = false
         coarsest(c);
         return false;
     }
-    if (level == 1 && level < d.max_level && !x_zero && cycle_bottom_available(d)) {
+    if (cycle_bottom_runs(d, level, x_zero)) {
         // levels 1 and 0 in one workgroup (the coarsest direct solve keeps its own launch)
         const bool rbgs = c.o->smoother == CMG_SMOOTH_RBGS;
         const int n = c.o->level_iters;
         // (the final x is written in place whatever the sweep count, so any count can prolong)
-        const bool push = push_up && !rbgs && n >= 1 && jacobi_push_available(d, 1);
+        const bool push = push_up && n >= 1 && jacobi_push_available(d, 1);
         double* rz = c.rz && !rbgs && n >= 1 ? c.rz + rz_offset(d, 1) : nullptr;
-        const bool fas1 = fas_save && !rbgs;
+        const bool fas1 = fas_save;
         if (c.o->coarsest_direct) {
             launch_cycle_bottom(d, 1, c.X, c.X0, c.B, c.C, c.s->Rr, c.s->P, rbgs, n, c.o->omega, 0, 0, fas1, false, nullptr,
                                 c.S, st);
@@ -983,8 +989,10 @@ bool cycle_step(const CycleCtx& c, int level, bool x_zero, bool fas_save = false
         smooth(c, level, c.o->level_iters, 0, x_zero, fas_save);
     }
     launch_residual_restrict(d, level, c.X, c.C, c.B, c.s->Rr, c.S, st);
-    // damped Jacobi: the coarser level's FAS save rides on its first pre-sweep
-    const bool fused = c.o->smoother == CMG_SMOOTH_JACOBI && c.o->level_iters >= 1 && fuse_fas_save_allowed();
+    // the coarser level's FAS save rides on its first pre-sweep (damped Jacobi), or on the
+    // workgroup that runs the bottom two levels
+    const bool fused = (c.o->smoother == CMG_SMOOTH_JACOBI || cycle_bottom_runs(d, level - 1, false)) &&
+                       c.o->level_iters >= 1 && fuse_fas_save_allowed();
     if (!fused) launch_fas_save(d, level - 1, c.X, c.C, c.B, c.X0, c.S, st);
     // In a PCG solve (the r.z fusion is on) the cycle's output is read on LEAF tiles only, so
     // the prolongation into the finest level is left to its post-sweeps, which compute it on
