@@ -38,6 +38,8 @@ struct LaunchList {
     std::vector<int32_t> order;   // the entries on the host (-1: padding)
 };
 
+constexpr int kDenseTiles = 512, kDenseWords = 64, kDenseNonleaf = 54, kDenseOct = 55;
+
 struct DevGrid {
     int N = 0;
     int num_levels = 0;
@@ -76,6 +78,11 @@ struct DevGrid {
     int bottom_entry[8] = {};
     int bottom_child[64] = {};
     unsigned long long bottom_ghost = 0;
+    // a complete level (8^l LEAF or NONLEAF tiles under a single root) of at most kDenseTiles
+    // tiles: kDenseWords words per subtree[l] entry (the 27 tiles around it, x slowest, -1
+    // outside the domain; their parents; at kDenseNonleaf a bit for each that is NONLEAF; at
+    // kDenseOct the tile's octant), else null
+    int32_t* dense[kMaxLevels] = {};
     LaunchList ghosts;                  // all GHOST tiles
     LaunchList leafghost;               // all LEAF and GHOST tiles
     LaunchList cyclezero;               // GHOST tiles and LEAF tiles below the finest level

@@ -63,26 +63,6 @@ __device__ __forceinline__ float staged_coef(const Lds<T, LQ>& s, int a, int i, 
     else return s.off[a][i];
 }
 
-// the entries of a coded level's table (the last one holds the tile spacing)
-template <int Q>
-constexpr int code_table() { return Q == 4 ? kWideCodes : kCodes; }
-
-// a cell word's code of the face coefficient on axis a: bits 8a+8.. (forms 2, 3) or 10a+2.. (form 4)
-template <int Q>
-__device__ __forceinline__ uint32_t word_code(uint32_t w, int a)
-{
-    if constexpr (Q == 4) return (w >> (10 * a + 2)) & 0x3ffu;
-    else return (w >> (8 * a + 8)) & 0xffu;
-}
-
-// a cell word's cell type: byte 0 (forms 2, 3), or 0..3 in bits 0-1 for 0, DIRICHLET, INTERIOR, NEUMANN (form 4)
-template <int Q>
-__device__ __forceinline__ uint8_t word_type(uint32_t w)
-{
-    if constexpr (Q == 4) return uint8_t((0x4210u >> (4 * (w & 3u))) & 0xfu);
-    else return uint8_t(w);
-}
-
 // a staged coefficient as FP32: FP32 as is, FP16 bits of c / h times h (exact: h is a
 // power of two times h0)
 __device__ __forceinline__ float lds_coef(float v, float) { return v; }
@@ -150,29 +130,6 @@ template <int NT>
 __device__ __forceinline__ int own_cell(int c)
 {
     return own_cell<NT>(c, int(threadIdx.x));
-}
-
-template <int N, typename E>
-struct alignas(N * sizeof(E)) Pack {
-    E v[N];
-};
-
-// N consecutive elements at p (aligned to N elements) in one access
-template <int N, typename E>
-__device__ __forceinline__ void vload(const E* __restrict__ p, E (&out)[N])
-{
-    const Pack<N, E> pk = *reinterpret_cast<const Pack<N, E>*>(p);
-#pragma unroll
-    for (int i = 0; i < N; ++i) out[i] = pk.v[i];
-}
-
-template <int N, typename E>
-__device__ __forceinline__ void vstore(E* __restrict__ p, const E (&in)[N])
-{
-    Pack<N, E> pk;
-#pragma unroll
-    for (int i = 0; i < N; ++i) pk.v[i] = in[i];
-    *reinterpret_cast<Pack<N, E>*>(p) = pk;
 }
 
 // four consecutive FP16 coefficients (quad q of the tile-major layout), back to FP32
@@ -1941,9 +1898,9 @@ __device__ __forceinline__ TileRec rec_tile_at(const int4* __restrict__ r, int t
 // on the first 256 threads.  Every step does the arithmetic of the per-pass kernel it
 // replaces (gs_color, jacobi, residual_restrict, fas_save, coarsest_tile, fas_prolong_v,
 // jacobi's r.z partial), so the results are bit-identical.
-// phase 1: level 1's FAS save, pre-smoothing, residual + restriction, the root's FAS save;
-// phase 2: the prolongation to level 1, its post-smoothing and the prolongation into level
-// 2; phase 3: both with the coarsest iterations (mu times) in between.
+// PHASE 1: level 1's FAS save, pre-smoothing, residual + restriction, the root's FAS save;
+// PHASE 2: the prolongation to level 1, its post-smoothing and the prolongation into level
+// 2; PHASE 3: both with the coarsest iterations (mu times) in between, `visits` times in a row.
 //
 // One CU does all of it, so a pass is bound by instruction issue (16 waves on 4 SIMDs) and
 // the chain LDS read - seven dependent fmas - division - LDS write - barrier.  Hence: a
@@ -1951,8 +1908,8 @@ __device__ __forceinline__ TileRec rec_tile_at(const int4* __restrict__ r, int t
 // pass, with no selects), the + face coefficients are registers, a division is a product
 // with the FP64 reciprocal of the diagonal, and the root's passes run on one wave per SIMD
 // with no memory traffic between them.  (MI355X, W-cycle settings with 10 coarsest
-// iterations and mu = 2, i.e. 8 passes on level 1 and 40 on the root: 19.6 us a visit, 0.17 us
-// a root pass; 44.2 us with every cell computed in every pass and the root's steps staged
+// iterations and mu = 2, i.e. 8 passes on level 1 and 40 on the root: 17.1 us a visit, 28.4 us
+// two visits in one launch, 0.17 us a root pass; 44.2 us a visit with every cell computed in every pass and the root's steps staged
 // through memory and computed twice, and another 9 us for level 1's FAS save and the
 // prolongation into level 2 in launches of their own.)
 struct BottomArgs {
@@ -1968,8 +1925,9 @@ struct BottomArgs {
     Coef C;
     float Rr, P, w;
     double omega;
-    int rbgs, iters, mu, coarsest_iters;
-    int phase, fas_save1, push;
+    int iters, mu, coarsest_iters;
+    int fas_save1, push;
+    int visits;          // PHASE 3: this many visits one after the other, the FAS save before the first
     double* rz;          // r.z partials of level 1's last post-sweep (Jacobi), or null
 };
 
@@ -1988,40 +1946,8 @@ struct BottomLds {
 __device__ __forceinline__ int bx(int i, int j, int k) { return (i + 1) * 324 + (j + 1) * 18 + (k + 1); }
 __device__ __forceinline__ int bc(int i, int j, int k) { return (i << 8) | (j << 4) | k; }
 
-// n / d for the FP64 reciprocal rd = 1 / d: the correctly rounded FP32 quotient.  The product
-// is within 2^-52 of n / d, and no quotient of two FP32 numbers lies within 2^-49 of the
-// midpoint of two neighbouring normal FP32 numbers.
-__device__ __forceinline__ float quotient(float n, double rd) { return float(double(n) * rd); }
-
-// one cell of a block kept in LDS: A x at LDS index c (strides si, sj, 1) with the face
-// coefficients in registers (neg_lap's order)
-__device__ __forceinline__ float block_lap(const float* x, int c, int si, int sj, float x0, const float (&cm)[3],
-                                           const float (&cp)[3], float d)
-{
-    const float v0 = x[c - si], v1 = x[c + si], v2 = x[c - sj], v3 = x[c + sj], v4 = x[c - 1], v5 = x[c + 1];
-    float r = x0 * d;
-    r = fmaf(cm[0], v0, r);
-    r = fmaf(cp[0], v1, r);
-    r = fmaf(cm[1], v2, r);
-    r = fmaf(cp[1], v3, r);
-    r = fmaf(cm[2], v4, r);
-    r = fmaf(cp[2], v5, r);
-    return d == 0 ? 0.0f : r;
-}
-
-// four consecutive cells, pairs swapped when odd: [2s] is then the pair's red cell, [2s + 1] its black one
-template <typename E>
-__device__ __forceinline__ void by_colour(E (&v)[4], bool odd)
-{
-#pragma unroll
-    for (int s = 0; s < 4; s += 2) {
-        const E a = v[s], b = v[s + 1];
-        v[s] = odd ? b : a;
-        v[s + 1] = odd ? a : b;
-    }
-}
-
-template <bool Q>
+// Q: the FP16 copies, SOR: red-black passes (else damped Jacobi), PHASE: see above
+template <bool Q, bool SOR, int PHASE>
 __global__ __launch_bounds__(1024) void cycle_bottom(TopoView tp, BottomArgs a, const double* __restrict__ S)
 {
     __shared__ BottomLds<Q> s;
@@ -2160,10 +2086,10 @@ __global__ __launch_bounds__(1024) void cycle_bottom(TopoView tp, BottomArgs a, 
             }
         }
 #pragma unroll
-        for (int c = 0; c < 4; ++c) rd[c] = 1.0 / double(d[c]);
+        for (int c = 0; c < 4; ++c) rd[c] = reciprocal(d[c]);
         if (rootw) {
 #pragma unroll
-            for (int e = 0; e < 2; ++e) rrd[e] = 1.0 / double(rdg[e]);
+            for (int e = 0; e < 2; ++e) rrd[e] = reciprocal(rdg[e]);
         }
     }
     const int n = a.iters;
@@ -2234,10 +2160,10 @@ __global__ __launch_bounds__(1024) void cycle_bottom(TopoView tp, BottomArgs a, 
     const int rv[2] = {cidx(ri, rj, rk0 + int(rodd)), cidx(ri, rj, rk0 + 1 - int(rodd))};
     float rxv[2] = {0.0f, 0.0f}, rbv[2] = {0.0f, 0.0f};
     auto root_lap = [&](int e) { return block_lap(s.rx, rl[e], 100, 10, rxv[e], rcm[e], rcp[e], rdg[e]); };
-    if (a.phase & 1) {
+    auto visit_down = [&](bool save1) {
         // pre-smoothing (order 0)
-        if (a.rbgs) {
-            if (a.fas_save1) {
+        if constexpr (SOR) {
+            if (save1) {
                 fas_save1();
                 __syncthreads();   // every read of x for the save is done before x changes
             }
@@ -2246,7 +2172,7 @@ __global__ __launch_bounds__(1024) void cycle_bottom(TopoView tp, BottomArgs a, 
                 colour_pass(Black{});
             }
         } else {
-            for (int it = 0; it < n; ++it) sweep(a.fas_save1 && it == 0, false);
+            for (int it = 0; it < n; ++it) sweep(save1 && it == 0, false);
         }
         // residual and restriction into the root (residual_restrict)
         __syncthreads();   // (res takes the place of the coefficients)
@@ -2275,7 +2201,7 @@ __global__ __launch_bounds__(1024) void cycle_bottom(TopoView tp, BottomArgs a, 
         }
         // level 1's x after the pre-smoothing (read back by phase 2 when the coarsest solve
         // runs in between; the jacobi ping-pong buffer is not written)
-        if (a.phase == 1) put4(a.X + v0, x);
+        if constexpr (PHASE == 1) put4(a.X + v0, x);
         __syncthreads();
         if (rootw) {
             const size_t rbase = size_t(root) * 512;
@@ -2307,8 +2233,8 @@ __global__ __launch_bounds__(1024) void cycle_bottom(TopoView tp, BottomArgs a, 
             }
         }
         __syncthreads();
-    }
-    if (a.phase == 3) {
+    };
+    auto visit_root = [&]() {
         // the coarsest iterations on the root (coarsest_tile)
         auto root_pass = [&](auto colour) {
             constexpr int e = decltype(colour)::value;
@@ -2321,9 +2247,9 @@ __global__ __launch_bounds__(1024) void cycle_bottom(TopoView tp, BottomArgs a, 
             }
             __syncthreads();
         };
-        const int it1 = a.rbgs ? a.coarsest_iters / 2 : a.coarsest_iters;
+        const int it1 = SOR ? a.coarsest_iters / 2 : a.coarsest_iters;
         for (int i = 0; i < a.mu; ++i) {
-            if (a.rbgs) {
+            if constexpr (SOR) {
                 for (int it = 0; it < it1; ++it) {
                     root_pass(Red{});
                     root_pass(Black{});
@@ -2359,18 +2285,35 @@ __global__ __launch_bounds__(1024) void cycle_bottom(TopoView tp, BottomArgs a, 
 #pragma unroll
             for (int e = 0; e < 2; ++e) a.X[rbase + rv[e]] = rxv[e];
         }
-    }
-    if (a.phase & 2) {
+    };
+    // level 2's cells below this thread's four: a 2 x 2 of rows of 8 cells of one child
+    const int oc = (li >> 2) | ((lj >> 2) << 1) | ((lk0 >> 2) << 2);
+    const int ch = PHASE != 1 && a.push ? a.child[8 * g + oc] : -1;
+    float pxf[4][8];
+    uint8_t pcf[4][8];
+    float px0[4];
+    auto push_loads = [&]() {
+        if (ch < 0) return;
+        vload<4>(a.X0 + v0, px0);
+#pragma unroll
+        for (int ab = 0; ab < 4; ++ab) {
+            const size_t fb = size_t(ch) * 512 + cidx(2 * (li & 3) + (ab >> 1), 2 * (lj & 3) + (ab & 1), 0);
+            vload<8>(a.X + fb, pxf[ab]);
+            vload<8>(tp.ctype + fb, pcf[ab]);
+        }
+    };
+    double acc = 0;
+    auto visit_up = [&]() {
         // the prolongation to level 1 (fas_prolong_v; no GHOST tile on a complete level 1)
         float cx[2], cx0[2];
-        if (a.phase == 2) {
+        if constexpr (PHASE == 2) {
             const size_t pb = size_t(root) * 512 + cidx(gi >> 1, gj >> 1, gk0 >> 1);
             const float2 xc = *reinterpret_cast<const float2*>(a.X + pb), x0c = *reinterpret_cast<const float2*>(a.X0 + pb);
             cx[0] = xc.x; cx[1] = xc.y;
             cx0[0] = x0c.x; cx0[1] = x0c.y;
         } else {
             // through LDS: x is there (with no coarsest iteration it is the restriction's, unmasked), X0 takes rb's place
-            const bool ran = a.mu > 0 && (a.rbgs ? a.coarsest_iters / 2 : a.coarsest_iters) > 0;
+            const bool ran = a.mu > 0 && (SOR ? a.coarsest_iters / 2 : a.coarsest_iters) > 0;
             if (rootw) {
 #pragma unroll
                 for (int e = 0; e < 2; ++e) {
@@ -2391,33 +2334,35 @@ __global__ __launch_bounds__(1024) void cycle_bottom(TopoView tp, BottomArgs a, 
             s.x[lx[c]] = x[c];
         }
         __syncthreads();
-        // post-smoothing (order 1); the last Jacobi sweep sums b.x = r.z.  The prolongation into
-        // level 2 follows; level 2's x and types are loaded before the last iteration
-        const int oc = (li >> 2) | ((lj >> 2) << 1) | ((lk0 >> 2) << 2);
-        const int ch = a.push ? a.child[8 * g + oc] : -1;
-        float pxf[4][8];
-        uint8_t pcf[4][8];
-        float px0[4];
-        double acc = 0;
+        // post-smoothing (order 1); the last Jacobi sweep sums b.x = r.z.  (A single visit loads
+        // level 2's cells for the prolongation before its last iteration; with several, the
+        // registers they take cost more than the wait)
         for (int it = 0; it < n; ++it) {
-            if (it == n - 1 && ch >= 0) {
-                vload<4>(a.X0 + v0, px0);
-#pragma unroll
-                for (int ab = 0; ab < 4; ++ab) {
-                    const size_t fb = size_t(ch) * 512 + cidx(2 * (li & 3) + (ab >> 1), 2 * (lj & 3) + (ab & 1), 0);
-                    vload<8>(a.X + fb, pxf[ab]);
-                    vload<8>(tp.ctype + fb, pcf[ab]);
-                }
-            }
-            if (a.rbgs) {
+            if (PHASE == 2 && it == n - 1) push_loads();
+            if constexpr (SOR) {
                 colour_pass(Black{});
                 colour_pass(Red{});
             } else {
                 acc = sweep(false, a.rz && it == n - 1);
             }
         }
+    };
+    if constexpr (PHASE == 3) {
+#pragma unroll 1
+        for (int visit = 0; visit < a.visits; ++visit) {
+            visit_down(a.fas_save1 && visit == 0);
+            visit_root();
+            visit_up();
+        }
+        push_loads();
+    } else if constexpr (PHASE == 1) {
+        visit_down(a.fas_save1);
+    } else {
+        visit_up();
+    }
+    if constexpr (PHASE != 1) {
         put4(a.X + v0, x);
-        if (a.rz) {
+        if (!SOR && a.rz) {
             // the tile's b.x partial, summed as block_sum sums a 128-thread workgroup's
             for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
             if ((threadIdx.x & 63) == 0) s.red[threadIdx.x >> 6] = acc;
@@ -3435,7 +3380,7 @@ bool cycle_bottom_available(const DevGrid& d)
 
 void launch_cycle_bottom(const DevGrid& d, int phase, float* X, float* X0, float* B, Coef C, float Rr, float P, bool rbgs,
                          int iters, double omega, int mu, int coarsest_iters, bool fas_save1, bool push, double* rz,
-                         const double* S, hipStream_t st)
+                         const double* S, hipStream_t st, int visits)
 {
     if (!cycle_bottom_available(d)) throw std::logic_error("cycle_bottom: levels 0 and 1 do not fit one workgroup");
     if (push && (iters < 1 || !jacobi_push_available(d, 1)))
@@ -3454,10 +3399,21 @@ void launch_cycle_bottom(const DevGrid& d, int phase, float* X, float* X0, float
     a.nonleaf0 = d.nonleaf[0].tiles;
     a.X = X; a.X0 = X0; a.B = B; a.C = C;
     a.Rr = Rr; a.P = P; a.w = float(omega); a.omega = omega;
-    a.rbgs = rbgs; a.iters = iters; a.mu = mu; a.coarsest_iters = coarsest_iters;
-    a.phase = phase; a.fas_save1 = fas_save1; a.push = push; a.rz = rz;
-    if (C.q[0]) k::cycle_bottom<true><<<1, 1024, 0, st>>>(view(d), a, run_flag(d, S));
-    else k::cycle_bottom<false><<<1, 1024, 0, st>>>(view(d), a, run_flag(d, S));
+    a.iters = iters; a.mu = mu; a.coarsest_iters = coarsest_iters;
+    a.fas_save1 = fas_save1; a.push = push; a.rz = rz; a.visits = phase == 3 ? visits : 1;
+    auto launch = [&](auto q, auto sor) {
+        constexpr bool Q = decltype(q)::value, SOR = decltype(sor)::value;
+        if (phase == 1) k::cycle_bottom<Q, SOR, 1><<<1, 1024, 0, st>>>(view(d), a, run_flag(d, S));
+        else if (phase == 2) k::cycle_bottom<Q, SOR, 2><<<1, 1024, 0, st>>>(view(d), a, run_flag(d, S));
+        else k::cycle_bottom<Q, SOR, 3><<<1, 1024, 0, st>>>(view(d), a, run_flag(d, S));
+    };
+    if (C.q[0]) {
+        if (rbgs) launch(std::true_type{}, std::true_type{});
+        else launch(std::true_type{}, std::false_type{});
+    } else {
+        if (rbgs) launch(std::false_type{}, std::true_type{});
+        else launch(std::false_type{}, std::false_type{});
+    }
 }
 
 bool coarsest_iterate_available(const DevGrid& d)

@@ -212,11 +212,20 @@ void launch_roi_flags(const DevGrid& d, const float* X, int subtree_level, int l
 
 // levels 0 and 1 fit one workgroup (level 0 one tile without neighbours, level 1 its 8
 // children) and forms bit 4 is clear: FASMuCycleStep at level 1 can run as
-// launch_cycle_bottom (phase 3; or phase 1, the coarsest solve, phase 2)
+// launch_cycle_bottom (phase 3, `visits` of them in a row; or phase 1, the coarsest solve, phase 2)
 bool cycle_bottom_available(const DevGrid& d);
 void launch_cycle_bottom(const DevGrid& d, int phase, float* X, float* X0, float* B, Coef C, float Rr, float P, bool rbgs,
                          int iters, double omega, int mu, int coarsest_iters, bool fas_save1, bool push, double* rz,
-                         const double* S, hipStream_t st);
+                         const double* S, hipStream_t st, int visits = 1);
+// a cycle's visit to a complete level (DevGrid::dense) in two launches (cmg_dense.hip): post
+// false the FAS save (when due), pre-smoothing, residual and restriction, x from X to T and
+// the saved right-hand side to BN; post true the prolongation from the level below,
+// post-smoothing, r.z partials (when rz) and the prolongation to the level above (when push),
+// x from T to X.  zero: x is 0 on the level.  One launch holds dense_visit_fits() iterations.
+bool dense_visit_fits(bool rbgs, int iters);
+void launch_dense_visit(const DevGrid& d, int level, bool post, float* X, float* T, float* B, float* BN, float* X0, Coef C,
+                        float Rr, float P, bool rbgs, int iters, double omega, bool zero, bool save, bool push, double* rz,
+                        const double* S, hipStream_t st);
 // level 0 is one tile without neighbours (and forms bit 4 is clear): its smoothing
 // iterations can run in one workgroup (launch_coarsest_iterate)
 bool coarsest_iterate_available(const DevGrid& d);

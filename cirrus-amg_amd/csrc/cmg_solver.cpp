@@ -37,6 +37,7 @@ struct cmg_solver {
     double* partial2 = nullptr;
     float* tmp = nullptr;          // Jacobi ping-pong buffer
     float* scratch = nullptr;      // cycle scratch of flexible CG (keeps Ap)
+    float* dense_b = nullptr;      // FAS-saved right-hand sides of the complete levels (launch_dense_visit)
     float* net_w = nullptr;        // learned tile smoother weights (7776 floats)
     unsigned int* lcount = nullptr;   // learned steps of the last solve: tiles judged, tiles kept
     uint16_t* q16 = nullptr;          // FP16 copies of the four coefficient channels / h (cycle_coef_fp16)
@@ -239,6 +240,7 @@ void dev_free(DevGrid& d)
     free_list(d.cyclezero_pull);
     free_list(d.finest_ghosts);
     for (int l = 0; l < kMaxLevels; ++l) {
+        if (d.dense[l]) (void)hipFree(d.dense[l]);
         free_list(d.subtree[l]);
         free_list(d.nonleaf[l]);
         free_list(d.prolong[l]);
@@ -391,6 +393,32 @@ void dev_upload(DevGrid& d, const Topology& topo)
             }
             d.bottom_ok = kids;
         }
+    }
+    for (int l = 1; d.root_alone && l < topo.num_levels() && l < kMaxLevels; ++l) {
+        const size_t n = size_t(1) << (3 * l);
+        if (n > kDenseTiles || sub[l].size() != n || pr[l].size() != n) break;
+        const int e = 1 << l;   // tiles along an edge
+        std::vector<int32_t> at(n);
+        auto place = [&](int x, int y, int z) { return (size_t(x) * e + y) * e + z; };
+        for (int t : sub[l]) at[place(topo.t_coord[t][0], topo.t_coord[t][1], topo.t_coord[t][2])] = t;
+        const std::vector<int32_t>& order = d.subtree[l].order;
+        std::vector<int32_t> tab(order.size() * kDenseWords, -1);
+        bool whole = order.size() == n;   // no padding entries
+        for (size_t i = 0; whole && i < order.size(); ++i) {
+            const int t = order[i];
+            int32_t* w = &tab[i * kDenseWords];
+            int32_t nonleaf = 0;
+            for (int o = 0; o < 27; ++o) {
+                const int x = topo.t_coord[t][0] + o / 9 - 1, y = topo.t_coord[t][1] + o / 3 % 3 - 1, z = topo.t_coord[t][2] + o % 3 - 1;
+                if (x < 0 || x >= e || y < 0 || y >= e || z < 0 || z >= e) continue;
+                w[o] = at[place(x, y, z)];
+                w[27 + o] = topo.parent[w[o]];
+                if (topo.t_type[w[o]] & NONLEAF) nonleaf |= 1 << o;
+            }
+            w[kDenseNonleaf] = nonleaf;
+            w[kDenseOct] = oct[t];
+        }
+        if (whole) up(d.dense[l], tab);
     }
     {
         int dev = 0, cus = 0;
@@ -926,6 +954,15 @@ bool cycle_bottom_runs(const DevGrid& d, int level, bool x_zero)
     return level == 1 && level < d.max_level && !x_zero && cycle_bottom_available(d);
 }
 
+// a cycle's visits to this level are two launches that each do all of a tile's passes
+bool dense_visit_runs(const cmg_solver* s, const cmg_solve_opts* o, int level)
+{
+    const DevGrid& d = s->g->dev;
+    return level >= 2 && level <= d.max_level && d.dense[level] && s->dense_b && s->family == CMG_SOLVER_AMG &&
+           !o->cycle_coef_fp16 && dense_visit_fits(o->smoother == CMG_SMOOTH_RBGS, o->level_iters) && fuse_rz_allowed() &&
+           !(level == d.max_level && o->learned);
+}
+
 void coarsest(const CycleCtx& c)
 {
     DevGrid& d = c.s->g->dev;
@@ -949,7 +986,8 @@ void coarsest(const CycleCtx& c)
 // has not run yet; the first pre-sweep does it
 // `push_up`: the caller prolongs to level + 1 next; the last post-sweep may do it
 // (returns whether it did)
-bool cycle_step(const CycleCtx& c, int level, bool x_zero, bool fas_save = false, bool push_up = false)
+// `visits`: that many visits in a row (the bottom of the cycle without the direct solve; else 1)
+bool cycle_step(const CycleCtx& c, int level, bool x_zero, bool fas_save = false, bool push_up = false, int visits = 1)
 {
     DevGrid& d = c.s->g->dev;
     hipStream_t st = d.stream;
@@ -974,11 +1012,16 @@ bool cycle_step(const CycleCtx& c, int level, bool x_zero, bool fas_save = false
                                 st);
         } else {
             launch_cycle_bottom(d, 3, c.X, c.X0, c.B, c.C, c.s->Rr, c.s->P, rbgs, n, c.o->omega, cycle_mu(c.o),
-                                c.o->coarsest_iters, fas1, push, rz, c.S, st);
+                                c.o->coarsest_iters, fas1, push, rz, c.S, st, visits);
         }
         return push;
     }
-    if (x_zero && level == d.max_level && c.o->learned && c.s->net_w) {
+    const bool rbgs = c.o->smoother == CMG_SMOOTH_RBGS;
+    const bool dense = dense_visit_runs(c.s, c.o, level);
+    if (dense) {
+        launch_dense_visit(d, level, false, c.X, c.s->tmp, c.B, c.s->dense_b, c.X0, c.C, c.s->Rr, c.s->P, rbgs,
+                           c.o->level_iters, c.o->omega, x_zero && !rbgs, fas_save, false, nullptr, c.S, st);
+    } else if (x_zero && level == d.max_level && c.o->learned && c.s->net_w) {
         // the learned tile smoother replaces the pre-smoothing of the finest level
         // (mode 2: runs before it); a tile whose residual it does not lower takes
         // the first Jacobi sweep instead
@@ -988,21 +1031,32 @@ bool cycle_step(const CycleCtx& c, int level, bool x_zero, bool fas_save = false
     } else {
         smooth(c, level, c.o->level_iters, 0, x_zero, fas_save);
     }
-    launch_residual_restrict(d, level, c.X, c.C, c.B, c.s->Rr, c.S, st);
-    // the coarser level's FAS save rides on its first pre-sweep (damped Jacobi), or on the
-    // workgroup that runs the bottom two levels
-    const bool fused = (c.o->smoother == CMG_SMOOTH_JACOBI || cycle_bottom_runs(d, level - 1, false)) &&
+    if (!dense) launch_residual_restrict(d, level, c.X, c.C, c.B, c.s->Rr, c.S, st);
+    // the coarser level's FAS save rides on its first pre-sweep (damped Jacobi), on its visit's
+    // first launch (a complete level), or on the workgroup that runs the bottom two levels
+    const bool fused = (!rbgs || dense_visit_runs(c.s, c.o, level - 1) || cycle_bottom_runs(d, level - 1, false)) &&
                        c.o->level_iters >= 1 && fuse_fas_save_allowed();
     if (!fused) launch_fas_save(d, level - 1, c.X, c.C, c.B, c.X0, c.S, st);
     // In a PCG solve (the r.z fusion is on) the cycle's output is read on LEAF tiles only, so
     // the prolongation into the finest level is left to its post-sweeps, which compute it on
     // the fly: no launch of its own and no sweep of the coarser level carrying it; the
     // finest GHOST tiles then keep their zeros.
-    const bool pull = c.rz && level == d.max_level && c.o->smoother == CMG_SMOOTH_JACOBI && c.o->level_iters >= 1 &&
-                      pull_prolong_allowed();
+    const bool pull = c.rz && level == d.max_level && !rbgs && c.o->level_iters >= 1 && pull_prolong_allowed();
     const int mu = cycle_mu(c.o);
     bool pushed = false;
-    for (int i = 0; i < mu; ++i) pushed = cycle_step(c, level - 1, false, fused && i == 0, !pull && i == mu - 1);
+    if (cycle_bottom_runs(d, level - 1, false) && !c.o->coarsest_direct) {
+        // the mu visits to the bottom in one launch
+        pushed = cycle_step(c, level - 1, false, fused, !pull && !dense, mu);
+    } else {
+        for (int i = 0; i < mu; ++i) pushed = cycle_step(c, level - 1, false, fused && i == 0, !pull && !dense && i == mu - 1);
+    }
+    if (dense) {
+        const bool push = push_up && level < d.max_level && d.push_ok[level + 1];
+        launch_dense_visit(d, level, true, c.X, c.s->tmp, c.B, c.s->dense_b, c.X0, c.C, c.s->Rr, c.s->P, rbgs,
+                           c.o->level_iters, c.o->omega, false, fas_save, push,
+                           c.rz && !rbgs ? c.rz + rz_offset(d, level) : nullptr, c.S, st);
+        return push;
+    }
     if (!pushed && !pull) launch_fas_prolong(d, level, c.X, c.X0, c.s->P, c.S, st);
     return smooth(c, level, c.o->level_iters, 1, false, false, push_up, pull);
 }
@@ -1199,7 +1253,7 @@ bool first_sweep_fusable(const cmg_solver* s, const cmg_solve_opts* o)
 {
     return s->family == CMG_SOLVER_AMG && (o->cycle == CMG_CYCLE_FAS_W || o->cycle == CMG_CYCLE_FAS_V) &&
            o->smoother == CMG_SMOOTH_JACOBI && o->level_iters >= 1 && !o->learned && !o->is_pure_neumann &&
-           s->g->dev.max_level >= 1 && fuse_first_sweep_allowed();
+           s->g->dev.max_level >= 1 && fuse_first_sweep_allowed() && !dense_visit_runs(s, o, s->g->dev.max_level);
 }
 
 // r.z can be summed by each level's last post-sweep over its LEAF tiles (whose b
@@ -1274,6 +1328,12 @@ void ensure_buffers(cmg_solver* s)
     if (!s->tmp) {
         s->tmp = dmalloc<float>(size_t(d.N) * kCells);
         HIPCHK(hipMemset(s->tmp, 0, size_t(d.N) * kCells * sizeof(float)));
+    }
+    if (!s->dense_b && s->family == CMG_SOLVER_AMG) {
+        int top = 0;
+        for (int l = 1; l < kMaxLevels; ++l)
+            if (d.dense[l]) top = l;
+        if (top) s->dense_b = dmalloc<float>(size_t(d.level_start[top + 1]) * kCells);
     }
     for (int c : {CH_X, CH_R, CH_P, CH_AP, CH_Z}) dev_channel(d, c);
     if (s->family == CMG_SOLVER_AMG)
@@ -1605,7 +1665,7 @@ void solver_destroy(cmg_solver* s)
 {
     if (!s) return;
     if (s->gexec) (void)hipGraphExecDestroy(s->gexec);
-    for (void* p : {(void*)s->S, (void*)s->partial, (void*)s->partial2, (void*)s->tmp, (void*)s->scratch, (void*)s->net_w,
+    for (void* p : {(void*)s->S, (void*)s->partial, (void*)s->partial2, (void*)s->tmp, (void*)s->scratch, (void*)s->dense_b, (void*)s->net_w,
                     (void*)s->lcount, (void*)s->q16, (void*)s->qbad, (void*)s->cw, (void*)s->clut, (void*)s->cws, (void*)s->czw,
                     (void*)s->x64, (void*)s->b64,
                     (void*)s->r64, (void*)s->inv0, (void*)s->cells0, (void*)s->zero0})
