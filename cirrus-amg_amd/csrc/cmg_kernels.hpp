@@ -154,8 +154,10 @@ int launch_diag_check(const DevGrid& d, Coef C, double* partial, hipStream_t st)
 // learned tile smoother (cmg_learn.hip)
 void launch_gather_tiles(const DevGrid& d, const int32_t* tiles, int n, const float* V, const float* D, int mode, float* out,
                          hipStream_t st);
-int launch_net_train(const float* X, const float* E, const int32_t* idx, int n, const float* W, float* gpart, double* lpart,
-                     int max_wg, bool bf16, hipStream_t st);
+// wpack: net_pack_floats() floats of workspace (the weights in the kernel's order)
+size_t net_pack_floats();
+int launch_net_train(const float* X, const float* E, const int32_t* idx, int n, const float* W, float* wpack, float* gpart,
+                     double* lpart, int max_wg, bool bf16, hipStream_t st);
 void launch_net_reduce(const float* gpart, const double* lpart, int nwg, int n, float* grad, double* loss, hipStream_t st);
 void launch_adam(float* W, float* M, float* V, const float* G, int t, float lr, float b1, float b2, float eps, hipStream_t st);
 void launch_net_infer(const DevGrid& d, const LaunchList& l, const float* R, const float* D, const float* W, float* Y,

@@ -37,7 +37,25 @@ __device__ __forceinline__ float bf16_round(float f)
     return __uint_as_float(u & 0xffff0000u);
 }
 
+typedef short bf16x4 __attribute__((ext_vector_type(4)));
+typedef short s16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ f32x4 mfma32(s16x8 a, s16x8 b, f32x4 c)
+{
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+
+// offset of tap t (0..26) in a volume of edge E
+__device__ __forceinline__ int tap_off(int t, int E) { return (t / 9 - 1) * E * E + ((t / 3) % 3 - 1) * E + (t % 3 - 1); }
+
 __device__ __forceinline__ uint16_t bf16_bits(float f) { return uint16_t(__float_as_uint(bf16_round(f)) >> 16); }
+
+__device__ __forceinline__ uint32_t pack_relu_bf16(float lo, float hi)
+{
+    return uint32_t(bf16_bits(lo > 0 ? lo : 0.0f)) | (uint32_t(bf16_bits(hi > 0 ? hi : 0.0f)) << 16);
+}
 
 // ---------------------------------------------------------------- gather ----
 // one halo'd 10^3 volume per tile of `list`: mode 0 the input feature r / D,
@@ -81,224 +99,468 @@ __global__ __launch_bounds__(256) void gather_tiles(TopoView tp, const int32_t* 
 }
 
 // ---------------------------------------------------------------- training ----
-// One workgroup (1024 threads) per chunk of tiles; x, a1, a2 and the loss
-// buffers live in LDS.  BF16: weights and activations are rounded to bfloat16
-// in the forward pass (FP32 accumulation); the backward pass is FP32.
+// One workgroup (512 threads, 8 wave64s) per chunk of tiles, everything of a tile in LDS.  BF16:
+// weights and activations are rounded to bfloat16 in the forward pass (FP32 accumulation);
+// the backward pass is FP32.
+//
+// Every convolution and weight gradient is a product on the matrix cores.  With 16 positions
+// of the volume (or the 27 taps) along N and K in steps of four,
+//   a1[co][p]     = sum over taps            W1[co][t] x[p + off t]             (K: 28 taps)
+//   a2[co][p]     = sum over taps, ci        W2[co][ci][t] a1[ci][p + off t]    (BF16: K: 2 taps x 16 ci)
+//   U[t][q]       = sum over ci              W3[ci][t] a2[ci][q],   y[p] = sum of U[t][p + off t]
+//   dW3[ci][t]    = sum over q               a2[ci][q] g[q - off t]
+//   g2[ci][q]     = sum over taps            W3[ci][t] g[q - off t]             (where a2 > 0)
+//   dW2[co][ci]   = sum over p, tap by tap   g2[co][p] a1[ci][p + off t]
+//   g1[ci][p]     = sum over taps, co        W2[co][ci][t] g2[co][p - off t]    (where a1 > 0)
+//   dW1[co][t]    = sum over p               g1[co][p] x[p + off t]
+// the FP32 ones on v_mfma_f32_16x16x4_f32, BF16's a2 on v_mfma_f32_16x16x32_bf16.  The two
+// products with 6.9 M multiplications, dW2 and g1, bound it: 13,600 of a tile's 16,000 FP32
+// MFMAs of 32 cycles, 53 us of a tile's time on the four SIMDs of a CU.  dW2's 27 taps are
+// dealt to four pairs of waves, seven accumulators each, a pair's waves taking half the
+// positions, so that one load of g2 serves seven products; g1 goes tap by tap over a wave's
+// eight blocks of positions, so that four registers hold the weights in use.  Volumes read
+// with an offset are zero-padded (x, g) or read through a mask of the taps that stay inside
+// (vm); channel rows are 1,012 floats apart, which puts 16 rows, and 4 rows of 16 positions,
+// on distinct banks.  (MI355X, 4,096 tiles, BF16: 2.03 ms, 127 us a tile, 92 TFLOP/s; 46.8 ms with
+// one FMA a multiplication on the vector units, every operand from LDS and the weights from
+// global memory.  Its gradients were 5e-8 from the 64-bit ones in FP32 mode, 8e-8 before.)
+constexpr int TS = 1012;   // floats from one channel's 1,000 positions to the next's (the rest 0)
+constexpr int NBLK = (NV + 15) / 16;   // 63 blocks of 16 positions
+
 struct TrainLds {
-    float x[NV];
-    float a1[NC * NV];
-    float a2[NC * NV];
-    float g[NV];    // y, then d = y - e, then dL/dy
-    float s[NV];    // interior Laplacian of d
-    double red[16];
+    float xp[1728], gp[1728], sp[1728];   // 12^3, zero rim: x; y - e, then dL/dy; the interior Laplacian of y - e
+    uint32_t vm[1008];                    // bit t: position + off t is inside the volume
+    uint16_t pt[1008];                    // the position's place in the 12^3 volumes
+    // FP32: a1 [16][TS]; BF16: a1 [2 halves of 8 channels][1000][8] and a2 [4 quarters of 4][1000][4],
+    // bfloat16; then g1 [16][TS]
+    float r0[16 * TS];
+    float g2[16 * TS];                    // FP32: a2, then g2; BF16: U[9][1000], then g2
+    float w1[7][64], w3[7][64];           // layers 1 and 3 as operands (row lane & 15, tap 4 s + lane / 16)
+    float w3u[3][4][64];                  // layer 3 for U (row tap 9 g + lane & 15, channel 4 kk + lane / 16)
+    double red[8];
 };
+static_assert(sizeof(TrainLds) <= 160 * 1024, "a CU's LDS");
+constexpr int kA2 = 32000, kZero = 64000;   // bytes into r0 (BF16): a2, 16 zero bytes
+
+// weights in the order the MFMA operands take them: [27 taps][4][64 lanes] for g1 (row ci = lane & 15,
+// column co = 4 kk + lane / 16), then for a2 the same by (co, ci), or with BF16 [14 tap pairs][64 lanes][8]
+constexpr int NPACK = 2 * 27 * 256;
 
 template <bool BF16>
-__global__ __launch_bounds__(1024) void net_train(const float* __restrict__ X, const float* __restrict__ E,
-                                                  const int32_t* __restrict__ idx, int n, int per_wg,
-                                                  const float* __restrict__ W, float* __restrict__ gpart,
-                                                  double* __restrict__ lpart)
+__global__ __launch_bounds__(256) void net_pack(const float* __restrict__ W, float* __restrict__ P)
 {
-    extern __shared__ unsigned char smem[];
+    const int e = blockIdx.x * 256 + threadIdx.x;
+    if (e < 6912) {
+        const int lane = e & 63, kk = (e >> 6) & 3, t = e >> 8;
+        const int r = lane & 15, c = 4 * kk + (lane >> 4);
+        const float b = W[OW2 + (c * NC + r) * 27 + t], f = W[OW2 + (r * NC + c) * 27 + t];
+        P[e] = BF16 ? bf16_round(b) : b;
+        if (!BF16) P[6912 + e] = f;
+    }
+    if (BF16 && e < 14 * 512) {
+        const int j = e & 7, lane = (e >> 3) & 63, m = e >> 9;
+        const int tap = 2 * m + (lane >> 5), ci = 8 * ((lane >> 4) & 1) + j;
+        reinterpret_cast<uint16_t*>(P + 6912)[e] = tap < 27 ? bf16_bits(W[OW2 + ((lane & 15) * NC + ci) * 27 + tap]) : uint16_t(0);
+    }
+}
+
+__device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+__device__ __forceinline__ float bf16_float(uint16_t v) { return __uint_as_float(uint32_t(v) << 16); }
+
+template <bool BF16>
+__global__ __launch_bounds__(512) void net_train(const float* __restrict__ X, const float* __restrict__ E,
+                                                 const int32_t* __restrict__ idx, int n, int per_wg,
+                                                 const float* __restrict__ W, const float* __restrict__ Wp,
+                                                 float* __restrict__ gpart, double* __restrict__ lpart)
+{
+    extern __shared__ __align__(16) unsigned char smem[];
     TrainLds& s = *reinterpret_cast<TrainLds*>(smem);
-    const int tid = threadIdx.x, nth = blockDim.x;
-    // this thread's weight-gradient accumulators: weights tid, tid + nth, ...
-    constexpr int WPT = (NW + 1023) / 1024;
-    float gacc[WPT];
+    unsigned char* const r0 = reinterpret_cast<unsigned char*>(s.r0);
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int col = lane & 15, grp = lane >> 4;
+    auto rnd = [](float v) { return BF16 ? bf16_round(v) : v; };
+    for (int e = tid; e < 1728; e += 512) s.xp[e] = s.gp[e] = s.sp[e] = 0.0f;
+    for (int e = tid; e < 16 * TS; e += 512) s.r0[e] = s.g2[e] = 0.0f;
+    for (int p = tid; p < 1008; p += 512) {
+        uint32_t m = 0;
+        const int i = p / 100, j = (p / 10) % 10, kk = p % 10;
+        for (int t = 0; t < 27; ++t) {
+            const int a = i + t / 9 - 1, b = j + (t / 3) % 3 - 1, c = kk + t % 3 - 1;
+            if (p < NV && unsigned(a) < 10u && unsigned(b) < 10u && unsigned(c) < 10u) m |= 1u << t;
+        }
+        s.vm[p] = m;
+        s.pt[p] = uint16_t(p < NV ? ((i + 1) * 12 + j + 1) * 12 + kk + 1 : 0);
+    }
+    float *const w1f = &s.w1[0][0], *const w3f = &s.w3[0][0], *const w3uf = &s.w3u[0][0][0];
+    for (int e = tid; e < 7 * 64; e += 512) {
+        const int t = 4 * (e >> 6) + ((e >> 4) & 3), r = e & 15;
+        w1f[e] = t < 27 ? rnd(W[r * 27 + t]) : 0.0f;
+        w3f[e] = t < 27 ? rnd(W[OW3 + r * 27 + t]) : 0.0f;
+    }
+    for (int e = tid; e < 12 * 64; e += 512) {
+        const int g = e >> 8, ci = 4 * ((e >> 6) & 3) + ((e >> 4) & 3), r = e & 15;
+        w3uf[e] = r < 9 ? rnd(W[OW3 + ci * 27 + 9 * g + r]) : 0.0f;
+    }
+    int o12[7], oc[2];   // offsets of the operands' taps 4 s + grp, and of the weight gradients' column taps
 #pragma unroll
-    for (int q = 0; q < WPT; ++q) gacc[q] = 0.0f;
+    for (int e = 0; e < 7; ++e) o12[e] = 4 * e + grp < 27 ? tap_off(4 * e + grp, 12) : 0;
+#pragma unroll
+    for (int e = 0; e < 2; ++e) oc[e] = 16 * e + col < 27 ? tap_off(16 * e + col, 12) : 0;
+    const int tap0 = 7 * (wave >> 1), half = wave & 1;   // the wave's share of dW2
+    // gradients of the workgroup's tiles
+    f32x4 G2[7], G3[2], G1[2];
+#pragma unroll
+    for (int m = 0; m < 7; ++m) G2[m] = f32x4{0, 0, 0, 0};
+#pragma unroll
+    for (int e = 0; e < 2; ++e) G3[e] = G1[e] = f32x4{0, 0, 0, 0};
     double lacc = 0;
+    __syncthreads();
+    uint32_t vmb[8];   // the masks of the wave's blocks of positions
+#pragma unroll
+    for (int b = 0; b < 8; ++b) vmb[b] = s.vm[min(16 * (wave + 8 * b) + col, 1007)];
+    auto block_pos = [&](int b) { return 16 * (wave + 8 * b) + col; };
+    // g[16 out][p] = sum over taps and 16 in of P[t][in][out] src[in][p + (or -) off t] for the
+    // wave's eight blocks; src channel rows of TS floats
+    auto conv16 = [&](const float* __restrict__ Pw, const float* src, bool flip, f32x4 (&acc)[8]) {
+#pragma unroll
+        for (int b = 0; b < 8; ++b) acc[b] = f32x4{0, 0, 0, 0};
+        float w[4];
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk) w[kk] = Pw[kk * 64 + lane];
+#pragma unroll 1
+        for (int t = 0; t < 27; ++t) {
+            float wn[4] = {w[0], w[1], w[2], w[3]};
+            if (t < 26) {
+#pragma unroll
+                for (int kk = 0; kk < 4; ++kk) wn[kk] = Pw[((t + 1) * 4 + kk) * 64 + lane];
+            }
+            const int u = flip ? 26 - t : t, off = tap_off(u, 10);
+#pragma unroll
+            for (int b = 0; b < 8; ++b) {
+                const float* q = src + grp * TS + ((vmb[b] >> u) & 1u ? block_pos(b) + off : NV);   // NV: zeros
+#pragma unroll
+                for (int kk = 0; kk < 4; ++kk) acc[b] = mfma4(w[kk], q[kk * 4 * TS], acc[b]);
+            }
+#pragma unroll
+            for (int kk = 0; kk < 4; ++kk) w[kk] = wn[kk];
+        }
+    };
     const int b0 = blockIdx.x * per_wg, b1 = min(n, b0 + per_wg);
     for (int bi = b0; bi < b1; ++bi) {
         const size_t b = idx ? size_t(idx[bi]) : size_t(bi);
-        for (int p = tid; p < NV; p += nth) s.x[p] = X[b * NV + p];
+        float ev[2];
+#pragma unroll
+        for (int m = 0; m < 2; ++m) {
+            const int p = tid + 512 * m;
+            ev[m] = p < NV ? E[b * NV + p] : 0.0f;
+            if (p < NV) s.xp[s.pt[p]] = rnd(X[b * NV + p]);
+        }
+        if (BF16 && tid < 4) reinterpret_cast<uint32_t*>(r0 + kZero)[tid] = 0u;
         __syncthreads();
         // layer 1
-        for (int o = tid; o < NC * NV; o += nth) {
-            const int co = o / NV, p = o % NV, i = p / 100, j = (p / 10) % 10, kk = p % 10;
-            float acc = 0.0f;
-            for (int t = 0; t < 27; ++t) {
-                const int a = i + t / 9 - 1, bb = j + (t / 3) % 3 - 1, c = kk + t % 3 - 1;
-                if (a < 0 || a > 9 || bb < 0 || bb > 9 || c < 0 || c > 9) continue;
-                float w = W[co * 27 + t], xv = s.x[vid(a, bb, c)];
-                if (BF16) { w = bf16_round(w); xv = bf16_round(xv); }
-                acc = fmaf(w, xv, acc);
+#pragma unroll 2
+        for (int bk = 0; bk < 8; ++bk) {
+            const int p = block_pos(bk), c = s.pt[min(p, 1007)];
+            f32x4 acc = {0, 0, 0, 0};
+#pragma unroll
+            for (int e = 0; e < 7; ++e) acc = mfma4(s.w1[e][lane], s.xp[max(c + o12[e], 0)], acc);
+            if (p < NV) {
+                if constexpr (BF16) {
+                    uint2 v;
+                    v.x = pack_relu_bf16(acc[0], acc[1]);
+                    v.y = pack_relu_bf16(acc[2], acc[3]);
+                    *reinterpret_cast<uint2*>(r0 + (grp >> 1) * 16000 + p * 16 + (grp & 1) * 8) = v;
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) s.r0[(4 * grp + e) * TS + p] = acc[e] > 0 ? acc[e] : 0.0f;
+                }
             }
-            acc = acc > 0 ? acc : 0.0f;
-            s.a1[o] = BF16 ? bf16_round(acc) : acc;
         }
         __syncthreads();
         // layer 2
-        for (int o = tid; o < NC * NV; o += nth) {
-            const int co = o / NV, p = o % NV, i = p / 100, j = (p / 10) % 10, kk = p % 10;
-            float acc = 0.0f;
-            for (int t = 0; t < 27; ++t) {
-                const int a = i + t / 9 - 1, bb = j + (t / 3) % 3 - 1, c = kk + t % 3 - 1;
-                if (a < 0 || a > 9 || bb < 0 || bb > 9 || c < 0 || c > 9) continue;
-                const int q = vid(a, bb, c);
-                for (int ci = 0; ci < NC; ++ci) {
-                    float w = W[OW2 + (co * NC + ci) * 27 + t];
-                    if (BF16) w = bf16_round(w);
-                    acc = fmaf(w, s.a1[ci * NV + q], acc);
+        {
+            f32x4 acc[8];
+            if constexpr (BF16) {
+#pragma unroll
+                for (int bk = 0; bk < 8; ++bk) acc[bk] = f32x4{0, 0, 0, 0};
+                const uint4* wq = reinterpret_cast<const uint4*>(Wp + 6912) + lane;
+                uint4 w = wq[0];
+#pragma unroll 1
+                for (int m = 0; m < 14; ++m) {
+                    const uint4 wn = m < 13 ? wq[64 * (m + 1)] : w;
+                    const int tap = 2 * m + (grp >> 1);   // (tap 27 has zero weights; its bit is never set)
+                    const int off = tap_off(tap, 10) * 16 + (grp & 1) * 16000;
+                    const uint32_t bit = 1u << tap;
+#pragma unroll
+                    for (int bk = 0; bk < 8; ++bk) {
+                        const int addr = (vmb[bk] & bit) ? block_pos(bk) * 16 + off : kZero;
+                        acc[bk] = mfma32(__builtin_bit_cast(s16x8, w), *reinterpret_cast<const s16x8*>(r0 + addr), acc[bk]);
+                    }
+                    w = wn;
+                }
+            } else {
+                conv16(Wp + 6912, s.r0, false, acc);
+            }
+#pragma unroll
+            for (int bk = 0; bk < 8; ++bk) {
+                const int p = block_pos(bk);
+                if (p >= NV) continue;
+                if constexpr (BF16) {
+                    uint2 v;
+                    v.x = pack_relu_bf16(acc[bk][0], acc[bk][1]);
+                    v.y = pack_relu_bf16(acc[bk][2], acc[bk][3]);
+                    *reinterpret_cast<uint2*>(r0 + kA2 + grp * 8000 + p * 8) = v;
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) s.g2[(4 * grp + e) * TS + p] = acc[bk][e] > 0 ? acc[bk][e] : 0.0f;
                 }
             }
-            acc = acc > 0 ? acc : 0.0f;
-            s.a2[o] = BF16 ? bf16_round(acc) : acc;
         }
         __syncthreads();
+        // a2 of channel c at position q
+        auto a2_at = [&](int c, int q) -> float {
+            if constexpr (BF16) return bf16_float(*reinterpret_cast<const uint16_t*>(r0 + kA2 + (c >> 2) * 8000 + q * 8 + (c & 3) * 2));
+            else return s.g2[c * TS + q];
+        };
         // layer 3 and d = y - e
-        for (int p = tid; p < NV; p += nth) {
-            const int i = p / 100, j = (p / 10) % 10, kk = p % 10;
-            float acc = 0.0f;
-            for (int t = 0; t < 27; ++t) {
-                const int a = i + t / 9 - 1, bb = j + (t / 3) % 3 - 1, c = kk + t % 3 - 1;
-                if (a < 0 || a > 9 || bb < 0 || bb > 9 || c < 0 || c > 9) continue;
-                const int q = vid(a, bb, c);
-                for (int ci = 0; ci < NC; ++ci) {
-                    float w = W[OW3 + ci * 27 + t];
-                    if (BF16) w = bf16_round(w);
-                    acc = fmaf(w, s.a2[ci * NV + q], acc);
+        {
+            float y[2] = {0.0f, 0.0f};
+            if constexpr (BF16) {
+#pragma unroll 1
+                for (int g = 0; g < 3; ++g) {
+#pragma unroll 2
+                    for (int bk = 0; bk < 8; ++bk) {
+                        const int q = block_pos(bk);
+                        f32x4 acc = {0, 0, 0, 0};
+#pragma unroll
+                        for (int kk = 0; kk < 4; ++kk) acc = mfma4(s.w3u[g][kk][lane], q < NV ? a2_at(4 * kk + grp, q) : 0.0f, acc);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+                            if (q < NV && 4 * grp + e < 9) s.g2[(4 * grp + e) * NV + q] = acc[e];
+                    }
+                    __syncthreads();
+#pragma unroll
+                    for (int m = 0; m < 2; ++m) {
+                        const int p = tid + 512 * m;
+                        const uint32_t ok = p < NV ? s.vm[p] >> (9 * g) : 0u;
+#pragma unroll
+                        for (int t = 0; t < 9; ++t)
+                            if ((ok >> t) & 1u) y[m] += s.g2[t * NV + p + tap_off(9 * g + t, 10)];
+                    }
+                    __syncthreads();
+                }
+            } else {
+#pragma unroll
+                for (int m = 0; m < 2; ++m) {
+                    const int p = tid + 512 * m;
+                    for (int t = 0; t < 27; ++t) {
+                        if (p >= NV || !((s.vm[p] >> t) & 1u)) continue;
+                        for (int ci = 0; ci < NC; ++ci) y[m] = fmaf(W[OW3 + ci * 27 + t], s.g2[ci * TS + p + tap_off(t, 10)], y[m]);
+                    }
                 }
             }
-            s.g[p] = acc - E[b * NV + p];
+#pragma unroll
+            for (int m = 0; m < 2; ++m)
+                if (tid + 512 * m < NV) s.gp[s.pt[tid + 512 * m]] = y[m] - ev[m];
         }
         __syncthreads();
         // s = interior Laplacian of d, loss
         double lt = 0;
-        for (int p = tid; p < NV; p += nth) {
-            const int i = p / 100, j = (p / 10) % 10, kk = p % 10;
+        for (int p = tid; p < NV; p += 512) {
+            const int i = p / 100, j = (p / 10) % 10, kk = p % 10, c = s.pt[p];
             float v = 0.0f;
             if (i >= 1 && i <= 8 && j >= 1 && j <= 8 && kk >= 1 && kk <= 8) {
-                v = 6.0f * s.g[p] - s.g[p - 100] - s.g[p + 100] - s.g[p - 10] - s.g[p + 10] - s.g[p - 1] - s.g[p + 1];
+                v = 6.0f * s.gp[c] - s.gp[c - 144] - s.gp[c + 144] - s.gp[c - 12] - s.gp[c + 12] - s.gp[c - 1] - s.gp[c + 1];
                 lt += double(v) * double(v);
             }
-            s.s[p] = v;
+            s.sp[c] = v;
         }
         lacc += lt;
         __syncthreads();
         // dL/dy = 2 Lap^T s / n
         const float sc = 2.0f / float(n);
-        for (int p = tid; p < NV; p += nth) {
-            const int i = p / 100, j = (p / 10) % 10, kk = p % 10;
-            float v = 6.0f * s.s[p];
-            if (i > 0) v -= s.s[p - 100];
-            if (i < 9) v -= s.s[p + 100];
-            if (j > 0) v -= s.s[p - 10];
-            if (j < 9) v -= s.s[p + 10];
-            if (kk > 0) v -= s.s[p - 1];
-            if (kk < 9) v -= s.s[p + 1];
-            s.g[p] = v * sc;
+        for (int p = tid; p < NV; p += 512) {
+            const int c = s.pt[p];
+            float v = 6.0f * s.sp[c];
+            v -= s.sp[c - 144];
+            v -= s.sp[c + 144];
+            v -= s.sp[c - 12];
+            v -= s.sp[c + 12];
+            v -= s.sp[c - 1];
+            v -= s.sp[c + 1];
+            s.gp[c] = v * sc;
         }
         __syncthreads();
-        // dL/dW3 (reads a2 before it is overwritten)
+        // dL/dW3 (a2 before it is overwritten): the waves take every eighth group of four positions
+        {
+            f32x4 acc[2] = {f32x4{0, 0, 0, 0}, f32x4{0, 0, 0, 0}};
+            for (int q0 = 4 * wave; q0 < NV; q0 += 32) {
+                const int q = q0 + grp, c = s.pt[q];
+                const float av = a2_at(col, q);
 #pragma unroll
-        for (int q = 0; q < WPT; ++q) {
-            const int wi = tid + q * nth;
-            if (wi < OW3 || wi >= NW) continue;
-            const int ci = (wi - OW3) / 27, t = (wi - OW3) % 27;
-            const int di = t / 9 - 1, dj = (t / 3) % 3 - 1, dk = t % 3 - 1;
-            float acc = 0.0f;
-            for (int p = 0; p < NV; ++p) {
-                const int i = p / 100 + di, j = (p / 10) % 10 + dj, kk = p % 10 + dk;
-                if (i < 0 || i > 9 || j < 0 || j > 9 || kk < 0 || kk > 9) continue;
-                acc = fmaf(s.g[p], s.a2[ci * NV + vid(i, j, kk)], acc);
+                for (int e = 0; e < 2; ++e) acc[e] = mfma4(av, s.gp[c - oc[e]], acc[e]);
             }
-            gacc[q] += acc;
+#pragma unroll
+            for (int e = 0; e < 2; ++e) G3[e] += acc[e];
         }
+        if (!BF16) __syncthreads();
+        // dL/da2 masked by ReLU'
+#pragma unroll 2
+        for (int bk = 0; bk < 8; ++bk) {
+            const int q = block_pos(bk), c = s.pt[min(q, 1007)];
+            f32x4 acc = {0, 0, 0, 0};
+#pragma unroll
+            for (int e = 0; e < 7; ++e) acc = mfma4(s.w3[e][lane], s.gp[max(c - o12[e], 0)], acc);
+            if (q < NV) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) s.g2[(4 * grp + e) * TS + q] = a2_at(4 * grp + e, q) > 0 ? acc[e] : 0.0f;
+            }
+        }
+        if (BF16 && tid < 16 * 12) s.g2[(tid / 12) * TS + NV + tid % 12] = 0.0f;   // (U was there)
         __syncthreads();
-        // dL/da2 masked by ReLU', in place of a2
-        for (int o = tid; o < NC * NV; o += nth) {
-            const int ci = o / NV, qv = o % NV, i = qv / 100, j = (qv / 10) % 10, kk = qv % 10;
-            float acc = 0.0f;
-            if (s.a2[o] > 0) {
-                for (int t = 0; t < 27; ++t) {
-                    const int a = i - (t / 9 - 1), bb = j - ((t / 3) % 3 - 1), c = kk - (t % 3 - 1);
-                    if (a < 0 || a > 9 || bb < 0 || bb > 9 || c < 0 || c > 9) continue;
-                    float w = W[OW3 + ci * 27 + t];
-                    if (BF16) w = bf16_round(w);
-                    acc = fmaf(w, s.g[vid(a, bb, c)], acc);
+        // dL/dW2: the wave's seven taps over its half of the positions
+        {
+            f32x4 acc[7];
+            int off[7];
+#pragma unroll
+            for (int m = 0; m < 7; ++m) {
+                acc[m] = f32x4{0, 0, 0, 0};
+                off[m] = tap_off(min(tap0 + m, 26), 10);
+            }
+            for (int p0 = 4 * half; p0 < NV; p0 += 8) {
+                const int p = p0 + grp;
+                const uint32_t ok = s.vm[p];
+                const float av = s.g2[col * TS + p];
+#pragma unroll
+                for (int m = 0; m < 7; ++m) {
+                    // 0 where the neighbour is outside (the load is inside LDS all the same)
+                    const uint32_t in = uint32_t(-int((ok >> (tap0 + m)) & 1u));
+                    uint32_t v;
+                    if constexpr (BF16)
+                        v = uint32_t(*reinterpret_cast<const uint16_t*>(r0 + (col >> 3) * 16000 + (p + off[m]) * 16 + (col & 7) * 2)) << 16;
+                    else
+                        v = __float_as_uint(*(reinterpret_cast<const float*>(r0) + col * TS + p + off[m]));
+                    acc[m] = mfma4(av, __uint_as_float(v & in), acc[m]);
                 }
             }
-            s.a2[o] = acc;
-        }
-        __syncthreads();
-        // dL/dW2
 #pragma unroll
-        for (int q = 0; q < WPT; ++q) {
-            const int wi = tid + q * nth;
-            if (wi < OW2 || wi >= OW3) continue;
-            const int co = (wi - OW2) / (NC * 27), ci = ((wi - OW2) / 27) % NC, t = (wi - OW2) % 27;
-            const int di = t / 9 - 1, dj = (t / 3) % 3 - 1, dk = t % 3 - 1;
-            float acc = 0.0f;
-            for (int p = 0; p < NV; ++p) {
-                const int i = p / 100 + di, j = (p / 10) % 10 + dj, kk = p % 10 + dk;
-                if (i < 0 || i > 9 || j < 0 || j > 9 || kk < 0 || kk > 9) continue;
-                acc = fmaf(s.a2[co * NV + p], s.a1[ci * NV + vid(i, j, kk)], acc);
-            }
-            gacc[q] += acc;
+            for (int m = 0; m < 7; ++m) G2[m] += acc[m];
         }
-        __syncthreads();
         // dL/da1 masked by ReLU', in place of a1
-        for (int o = tid; o < NC * NV; o += nth) {
-            const int ci = o / NV, qv = o % NV, i = qv / 100, j = (qv / 10) % 10, kk = qv % 10;
-            float acc = 0.0f;
-            if (s.a1[o] > 0) {
-                for (int t = 0; t < 27; ++t) {
-                    const int a = i - (t / 9 - 1), bb = j - ((t / 3) % 3 - 1), c = kk - (t % 3 - 1);
-                    if (a < 0 || a > 9 || bb < 0 || bb > 9 || c < 0 || c > 9) continue;
-                    const int p = vid(a, bb, c);
-                    for (int co = 0; co < NC; ++co) {
-                        float w = W[OW2 + (co * NC + ci) * 27 + t];
-                        if (BF16) w = bf16_round(w);
-                        acc = fmaf(w, s.a2[co * NV + p], acc);
+        {
+            f32x4 acc[8];
+            conv16(Wp, s.g2, true, acc);
+#pragma unroll
+            for (int bk = 0; bk < 8; ++bk) {
+                const int p = block_pos(bk);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    bool on = false;
+                    if (p < NV) {
+                        if constexpr (BF16)
+                            on = bf16_float(*reinterpret_cast<const uint16_t*>(r0 + (grp >> 1) * 16000 + p * 16 + (grp & 1) * 8 + 2 * e)) > 0;
+                        else
+                            on = s.r0[(4 * grp + e) * TS + p] > 0;
                     }
+                    acc[bk][e] = on ? acc[bk][e] : 0.0f;
                 }
             }
-            s.a1[o] = acc;
+            __syncthreads();
+#pragma unroll
+            for (int bk = 0; bk < 8; ++bk) {
+                const int p = block_pos(bk);
+                if (p >= NV) continue;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) s.r0[(4 * grp + e) * TS + p] = acc[bk][e];
+            }
         }
         __syncthreads();
         // dL/dW1
+        {
+            f32x4 acc[2] = {f32x4{0, 0, 0, 0}, f32x4{0, 0, 0, 0}};
+            for (int p0 = 4 * wave; p0 < NV; p0 += 32) {
+                const int p = p0 + grp, c = s.pt[p];
+                const float av = s.r0[col * TS + p];
 #pragma unroll
-        for (int q = 0; q < WPT; ++q) {
-            const int wi = tid + q * nth;
-            if (wi >= OW2) continue;
-            const int co = wi / 27, t = wi % 27;
-            const int di = t / 9 - 1, dj = (t / 3) % 3 - 1, dk = t % 3 - 1;
-            float acc = 0.0f;
-            for (int p = 0; p < NV; ++p) {
-                const int i = p / 100 + di, j = (p / 10) % 10 + dj, kk = p % 10 + dk;
-                if (i < 0 || i > 9 || j < 0 || j > 9 || kk < 0 || kk > 9) continue;
-                float xv = s.x[vid(i, j, kk)];
-                if (BF16) xv = bf16_round(xv);
-                acc = fmaf(s.a1[co * NV + p], xv, acc);
+                for (int e = 0; e < 2; ++e) acc[e] = mfma4(av, s.xp[c + oc[e]], acc[e]);
             }
-            gacc[q] += acc;
+#pragma unroll
+            for (int e = 0; e < 2; ++e) G1[e] += acc[e];
         }
         __syncthreads();
     }
+    // the workgroup's gradients: dW2 from the two halves, dW1 and dW3 from the eight waves
+    float* out = gpart + size_t(blockIdx.x) * NW;
+    if (half) {
 #pragma unroll
-    for (int q = 0; q < WPT; ++q) {
-        const int wi = tid + q * nth;
-        if (wi < NW) gpart[size_t(blockIdx.x) * NW + wi] = gacc[q];
+        for (int m = 0; m < 7; ++m)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) s.r0[((wave >> 1) * 7 + m) * 256 + (4 * grp + e) * 16 + col] = G2[m][e];
+    }
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int at = wave * 512 + (4 * grp + e) * 32 + 16 * k + col;
+            s.g2[at] = G1[k][e];
+            s.g2[4096 + at] = G3[k][e];
+        }
+    __syncthreads();
+    if (!half) {
+#pragma unroll
+        for (int m = 0; m < 7; ++m) {
+            const int t = tap0 + m;
+            if (t >= 27) continue;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int co = 4 * grp + e;
+                out[OW2 + (co * NC + col) * 27 + t] = G2[m][e] + s.r0[((wave >> 1) * 7 + m) * 256 + co * 16 + col];
+            }
+        }
+    }
+    for (int e = tid; e < 432; e += 512) {
+        const int at = (e / 27) * 32 + e % 27;
+        float v1 = 0.0f, v3 = 0.0f;
+        for (int w = 0; w < 8; ++w) {
+            v1 += s.g2[w * 512 + at];
+            v3 += s.g2[4096 + w * 512 + at];
+        }
+        out[e] = v1;
+        out[OW3 + e] = v3;
     }
     const double lb = block_sum(lacc, s.red);
     if (tid == 0) lpart[blockIdx.x] = lb;
 }
 
-// grad[w] = sum over workgroups of the partials (fixed order, FP64); loss likewise
-__global__ __launch_bounds__(256) void net_reduce(const float* __restrict__ gpart, const double* __restrict__ lpart, int nwg,
-                                                  int n, float* __restrict__ grad, double* __restrict__ loss)
+// grad[w] = sum over workgroups of the partials (fixed order, FP64); loss likewise.  Few waves
+// with a long sum each: 32 partials are in flight at a time (MI355X, 256 workgroups:
+// 10 us, 72 us with one load in flight a thread)
+__global__ __launch_bounds__(64) void net_reduce(const float* __restrict__ gpart, const double* __restrict__ lpart, int nwg,
+                                                 int n, float* __restrict__ grad, double* __restrict__ loss)
 {
     const int wi = blockIdx.x * blockDim.x + threadIdx.x;
     if (wi < NW) {
         double acc = 0;
-        for (int g = 0; g < nwg; ++g) acc += double(gpart[size_t(g) * NW + wi]);
+        int g = 0;
+        for (; g + 32 <= nwg; g += 32) {
+            float v[32];
+#pragma unroll
+            for (int e = 0; e < 32; ++e) v[e] = gpart[size_t(g + e) * NW + wi];
+#pragma unroll
+            for (int e = 0; e < 32; ++e) acc += double(v[e]);
+        }
+        for (; g < nwg; ++g) acc += double(gpart[size_t(g) * NW + wi]);
         grad[wi] = float(acc);
     }
-    if (wi == 0) {
+    if (blockIdx.x == gridDim.x - 1) {
+        // the loss, its partials read a wave at a time
         double l = 0;
-        for (int g = 0; g < nwg; ++g) l += lpart[g];
-        *loss = l / double(n);
+        for (int g0 = 0; g0 < nwg; g0 += 64) {
+            const double v = g0 + int(threadIdx.x) < nwg ? lpart[g0 + threadIdx.x] : 0.0;
+            for (int e = 0; e < 64; ++e) l += __shfl(v, e, 64);
+        }
+        if (threadIdx.x == 0) *loss = l / double(n);
     }
 }
 
@@ -344,10 +606,6 @@ __global__ __launch_bounds__(256) void adam(float* __restrict__ W, float* __rest
 //   [36032, 68032)    a2, bf16
 //   [68032, 71488)    x on the zero-padded 12^3 volume, bf16 (edges and
 //                     corners of the 10^3 volume and the padding stay 0)
-typedef short bf16x4 __attribute__((ext_vector_type(4)));
-typedef short s16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int IL_A1 = 0, IL_ZERO = 36000, IL_A2 = 36032, IL_X = 68032, IL_BYTES = 71488;
 constexpr int IN_PT = 4;   // input cells per thread (896 = 512 own + 384 halo, 256 threads)
@@ -409,20 +667,6 @@ __device__ __forceinline__ void infer_issue(InferIn& in, const TopoView& tp, int
         }
     }
 }
-constexpr int NBLK = (NV + 15) / 16;   // 63 blocks of 16 positions
-
-__device__ __forceinline__ uint32_t pack_relu_bf16(float lo, float hi)
-{
-    return uint32_t(bf16_bits(lo > 0 ? lo : 0.0f)) | (uint32_t(bf16_bits(hi > 0 ? hi : 0.0f)) << 16);
-}
-
-__device__ __forceinline__ f32x4 mfma32(s16x8 a, s16x8 b, f32x4 c)
-{
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-}
-
-// offset of tap t (0..26) in a volume of edge E
-__device__ __forceinline__ int tap_off(int t, int E) { return (t / 9 - 1) * E * E + ((t / 3) % 3 - 1) * E + (t % 3 - 1); }
 
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void net_infer(TopoView tp, const int32_t* __restrict__ tiles, int n,
                                                  const float* __restrict__ R, const float* __restrict__ D,
@@ -620,8 +864,8 @@ void launch_gather_tiles(const DevGrid& d, const int32_t* tiles, int n, const fl
     k::gather_tiles<<<n, 256, 0, st>>>(view(d), tiles, n, V, D, mode, out);
 }
 
-int launch_net_train(const float* X, const float* E, const int32_t* idx, int n, const float* W, float* gpart, double* lpart,
-                     int max_wg, bool bf16, hipStream_t st)
+int launch_net_train(const float* X, const float* E, const int32_t* idx, int n, const float* W, float* wpack, float* gpart,
+                     double* lpart, int max_wg, bool bf16, hipStream_t st)
 {
     if (n <= 0) return 0;
     const int nwg = std::max(1, std::min(max_wg, n));
@@ -636,14 +880,21 @@ int launch_net_train(const float* X, const float* E, const int32_t* idx, int n, 
         return true;
     }();
     (void)attr;
-    if (bf16) k::net_train<true><<<used, 1024, lds, st>>>(X, E, idx, n, per, W, gpart, lpart);
-    else k::net_train<false><<<used, 1024, lds, st>>>(X, E, idx, n, per, W, gpart, lpart);
+    if (bf16) {
+        k::net_pack<true><<<28, 256, 0, st>>>(W, wpack);
+        k::net_train<true><<<used, 512, lds, st>>>(X, E, idx, n, per, W, wpack, gpart, lpart);
+    } else {
+        k::net_pack<false><<<28, 256, 0, st>>>(W, wpack);
+        k::net_train<false><<<used, 512, lds, st>>>(X, E, idx, n, per, W, wpack, gpart, lpart);
+    }
     return used;
 }
 
+size_t net_pack_floats() { return size_t(k::NPACK); }
+
 void launch_net_reduce(const float* gpart, const double* lpart, int nwg, int n, float* grad, double* loss, hipStream_t st)
 {
-    k::net_reduce<<<(k::NW + 255) / 256, 256, 0, st>>>(gpart, lpart, nwg, n, grad, loss);
+    k::net_reduce<<<(k::NW + 63) / 64, 64, 0, st>>>(gpart, lpart, nwg, n, grad, loss);
 }
 
 void launch_adam(float* W, float* M, float* V, const float* G, int t, float lr, float b1, float b2, float eps, hipStream_t st)

@@ -1989,6 +1989,7 @@ struct cmg_trainer {
     float *X = nullptr, *E = nullptr;
     float *W = nullptr, *M = nullptr, *V = nullptr, *G = nullptr;
     float* gpart = nullptr;
+    float* wpack = nullptr;   // the weights in the training kernel's order
     double *lpart = nullptr, *loss = nullptr;
     int32_t* idx = nullptr;
     int max_wg = 0;
@@ -2030,6 +2031,7 @@ cmg_status trainer_create(int capacity, uint64_t seed, cmg_trainer** out)
         HIPCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
         t->max_wg = std::max(1, cus);
         t->gpart = dmalloc<float>(size_t(t->max_wg) * kNetWeights);
+        t->wpack = dmalloc<float>(net_pack_floats());
         t->lpart = dmalloc<double>(size_t(t->max_wg));
         t->loss = dmalloc<double>(1);
         t->idx = dmalloc<int32_t>(size_t(capacity));
@@ -2060,7 +2062,7 @@ int trainer_size(const cmg_trainer* t) { return t ? t->size : 0; }
 void trainer_destroy(cmg_trainer* t)
 {
     if (!t) return;
-    for (void* p : {(void*)t->X, (void*)t->E, (void*)t->W, (void*)t->M, (void*)t->V, (void*)t->G, (void*)t->gpart,
+    for (void* p : {(void*)t->X, (void*)t->E, (void*)t->W, (void*)t->M, (void*)t->V, (void*)t->G, (void*)t->gpart, (void*)t->wpack,
                     (void*)t->lpart, (void*)t->loss, (void*)t->idx})
         if (p) (void)hipFree(p);
     if (t->stream) (void)hipStreamDestroy(t->stream);
@@ -2122,7 +2124,7 @@ cmg_status trainer_loss_grad(cmg_trainer* t, int first, int n, int bf16, double*
     if (!t || first < 0 || n <= 0 || first + n > t->size || !loss) return CMG_ERR_BAD_ARG;
     CMG_TRY({
         const int used = launch_net_train(t->X + size_t(first) * kNetVolume, t->E + size_t(first) * kNetVolume, nullptr, n,
-                                          t->W, t->gpart, t->lpart, t->max_wg, bf16 != 0, t->stream);
+                                          t->W, t->wpack, t->gpart, t->lpart, t->max_wg, bf16 != 0, t->stream);
         launch_net_reduce(t->gpart, t->lpart, used, n, t->G, t->loss, t->stream);
         HIPCHK(hipMemcpyAsync(loss, t->loss, sizeof(double), hipMemcpyDeviceToHost, t->stream));
         if (grad) HIPCHK(hipMemcpyAsync(grad, t->G, kNetWeights * sizeof(float), hipMemcpyDeviceToHost, t->stream));
@@ -2147,7 +2149,7 @@ cmg_status trainer_step(cmg_trainer* t, int batch, float lr, int bf16, double* l
         HIPCHK(hipMemcpyAsync(t->idx, t->perm.data() + t->perm_pos, size_t(batch) * sizeof(int32_t), hipMemcpyHostToDevice,
                               t->stream));
         t->perm_pos += batch;
-        const int used = launch_net_train(t->X, t->E, t->idx, batch, t->W, t->gpart, t->lpart, t->max_wg, bf16 != 0, t->stream);
+        const int used = launch_net_train(t->X, t->E, t->idx, batch, t->W, t->wpack, t->gpart, t->lpart, t->max_wg, bf16 != 0, t->stream);
         launch_net_reduce(t->gpart, t->lpart, used, batch, t->G, t->loss, t->stream);
         launch_adam(t->W, t->M, t->V, t->G, ++t->step, lr, 0.9f, 0.999f, 1e-8f, t->stream);
         if (loss) HIPCHK(hipMemcpyAsync(loss, t->loss, sizeof(double), hipMemcpyDeviceToHost, t->stream));
