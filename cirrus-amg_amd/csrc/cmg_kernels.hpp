@@ -235,6 +235,11 @@ bool coarsest_iterate_available(const DevGrid& d);
 // (w unused); else `iters` damped-Jacobi sweeps with weight w (omega, iters2, order unused)
 void launch_coarsest_iterate(const DevGrid& d, float* X, Coef C, const float* B, bool rbgs, int iters, int iters2, int order,
                              double omega, float w, const double* S, hipStream_t st);
+// the inverse of a symmetric n x n matrix (n <= 4096: `shift` everywhere plus the given entries,
+// row << 16 | column, no place twice) into inv (cmg_inverse.hip); false when a pivot of the
+// elimination is not positive or nearly 0 (inv is then not an inverse).  Synchronises the stream.
+bool device_inverse(int n, double shift, const std::vector<uint32_t>& rc, const std::vector<double>& v, double* inv,
+                    hipStream_t st);
 void launch_coarse_direct(const double* inv, const int32_t* cells, int n, const int32_t* zero_cells, int nz, float* X,
                           const float* B, const double* S, hipStream_t st);
 

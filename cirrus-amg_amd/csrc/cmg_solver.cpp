@@ -749,9 +749,72 @@ Coef solver_coef(const cmg_solver* s)
     return c;
 }
 
+// a matrix by rows of (column, value)
+using MatrixRows = std::vector<std::vector<std::pair<int, double>>>;
+
+bool symmetric(const MatrixRows& rows)
+{
+    for (size_t r = 0; r < rows.size(); ++r)
+        for (const auto& e : rows[r]) {
+            bool same = false;
+            for (const auto& o : rows[size_t(e.first)]) same = same || (o.first == int(r) && o.second == e.second);
+            if (!same) return false;
+        }
+    return true;
+}
+
+bool inverse_on_device(int n, double shift, const MatrixRows& rows, double* inv, hipStream_t st)
+{
+    std::vector<uint32_t> rc;
+    std::vector<double> v;
+    for (int r = 0; r < n; ++r)
+        for (const auto& e : rows[r]) {
+            rc.push_back(uint32_t(r) << 16 | uint32_t(e.first));
+            v.push_back(e.second);
+        }
+    return device_inverse(n, shift, rc, v, inv, st);
+}
+
+// Gauss-Jordan inverse with partial pivoting of the rows plus `shift` everywhere
+std::vector<double> pivoted_inverse(int n, double shift, const MatrixRows& rows)
+{
+    std::vector<double> A(size_t(n) * n, shift), inv(size_t(n) * n, 0.0);
+    for (int r = 0; r < n; ++r)
+        for (const auto& e : rows[r]) A[size_t(r) * n + e.first] += e.second;
+    for (int i = 0; i < n; ++i) inv[size_t(i) * n + i] = 1.0;
+    for (int k = 0; k < n; ++k) {
+        int piv = k;
+        for (int i = k + 1; i < n; ++i)
+            if (std::fabs(A[size_t(i) * n + k]) > std::fabs(A[size_t(piv) * n + k])) piv = i;
+        if (A[size_t(piv) * n + k] == 0) throw std::runtime_error("singular level-0 operator");
+        if (piv != k)
+            for (int j = 0; j < n; ++j) {
+                std::swap(A[size_t(k) * n + j], A[size_t(piv) * n + j]);
+                std::swap(inv[size_t(k) * n + j], inv[size_t(piv) * n + j]);
+            }
+        const double dk = 1.0 / A[size_t(k) * n + k];
+        for (int j = 0; j < n; ++j) {
+            A[size_t(k) * n + j] *= dk;
+            inv[size_t(k) * n + j] *= dk;
+        }
+        // rows are independent once row k is scaled
+#pragma omp parallel for schedule(static) if (n >= 256)
+        for (int i = 0; i < n; ++i) {
+            if (i == k) continue;
+            const double f = A[size_t(i) * n + k];
+            if (f == 0) continue;
+            for (int j = 0; j < n; ++j) {
+                A[size_t(i) * n + j] -= f * A[size_t(k) * n + j];
+                inv[size_t(i) * n + j] -= f * inv[size_t(k) * n + j];
+            }
+        }
+    }
+    return inv;
+}
+
 // dense FP64 inverse of the level-0 operator on its INTERIOR cells, probed
 // cell by cell with the same halo rules as the device stencil (level 0 has no
-// ghosts); Gauss-Jordan with partial pivoting.  For a pure-Neumann system the
+// ghosts).  For a pure-Neumann system the
 // constant null space is removed by adding mean(D)/n * 1 1^T.
 void build_direct(cmg_solver* s, bool pure_neumann)
 {
@@ -785,16 +848,26 @@ void build_direct(cmg_solver* s, bool pure_neumann)
         }
     const int n = int(cells.size());
     if (n > 4096) throw std::runtime_error("level-0 system too large for the dense direct solve");
-    std::vector<double> A(size_t(n) * n, 0.0);
+    // the matrix's entries, row by row
+    std::vector<std::vector<std::pair<int, double>>> rows(n);
     auto unknown = [&](int t, int v) -> int {
         if (t < lo || t >= hi) return -1;
         return T[size_t(t) * kCells + v] == INTERIOR ? map[size_t(t - lo) * kCells + v] : -1;
     };
+    double shift = 0;
     for (int r = 0; r < n; ++r) {
         const int t = cells[r] / kCells, v = cells[r] % kCells;
         const double D = C[3][cells[r]];
         if (D == 0) continue;
-        A[size_t(r) * n + r] += D;
+        auto add = [&](int c, double x) {
+            for (auto& e : rows[r])
+                if (e.first == c) {
+                    e.second += x;
+                    return;
+                }
+            rows[r].push_back({c, x});
+        };
+        add(r, D);
         const int l[3] = {v >> 6, (v >> 3) & 7, v & 7};
         for (int a = 0; a < 3; ++a)
             for (int sg = -1; sg <= 1; sg += 2) {
@@ -812,55 +885,36 @@ void build_direct(cmg_solver* s, bool pure_neumann)
                 else off = C[a][size_t(tt) * kCells + nv];
                 if (tt < 0) continue;
                 const int c = unknown(tt, nv);
-                if (c >= 0) A[size_t(r) * n + c] += off;
+                if (c >= 0) add(c, off);
             }
     }
     if (pure_neumann && n > 0) {
-        double md = 0;
-        for (int r = 0; r < n; ++r) md += A[size_t(r) * n + r];
-        md /= double(n) * double(n);
-        for (auto& a : A) a += md;
+        for (int r = 0; r < n; ++r)
+            for (auto& e : rows[r])
+                if (e.first == r) shift += e.second;
+        shift /= double(n) * double(n);
     }
-    // Gauss-Jordan inverse
-    std::vector<double> inv(size_t(n) * n, 0.0);
-    for (int i = 0; i < n; ++i) inv[size_t(i) * n + i] = 1.0;
-    for (int k = 0; k < n; ++k) {
-        int piv = k;
-        for (int i = k + 1; i < n; ++i)
-            if (std::fabs(A[size_t(i) * n + k]) > std::fabs(A[size_t(piv) * n + k])) piv = i;
-        if (A[size_t(piv) * n + k] == 0) throw std::runtime_error("singular level-0 operator");
-        if (piv != k)
-            for (int j = 0; j < n; ++j) {
-                std::swap(A[size_t(k) * n + j], A[size_t(piv) * n + j]);
-                std::swap(inv[size_t(k) * n + j], inv[size_t(piv) * n + j]);
-            }
-        const double dk = 1.0 / A[size_t(k) * n + k];
-        for (int j = 0; j < n; ++j) {
-            A[size_t(k) * n + j] *= dk;
-            inv[size_t(k) * n + j] *= dk;
+    double* const dinv = dmalloc<double>(size_t(n) * n);
+    try {
+        // on the device when the matrix is symmetric and its elimination meets positive pivots only
+        // (every operator assembled here); else with partial pivoting on the host
+        if (!(n > 0 && symmetric(rows) && inverse_on_device(n, shift, rows, dinv, d.stream))) {
+            const std::vector<double> inv = pivoted_inverse(n, shift, rows);
+            if (n) HIPCHK(hipMemcpy(dinv, inv.data(), inv.size() * sizeof(double), hipMemcpyHostToDevice));
         }
-        // rows are independent once row k is scaled
-#pragma omp parallel for schedule(static) if (n >= 256)
-        for (int i = 0; i < n; ++i) {
-            if (i == k) continue;
-            const double f = A[size_t(i) * n + k];
-            if (f == 0) continue;
-            for (int j = 0; j < n; ++j) {
-                A[size_t(i) * n + j] -= f * A[size_t(k) * n + j];
-                inv[size_t(i) * n + j] -= f * inv[size_t(k) * n + j];
-            }
-        }
+    } catch (...) {
+        (void)hipFree(dinv);
+        throw;
     }
     if (s->inv0) (void)hipFree(s->inv0);
     if (s->cells0) (void)hipFree(s->cells0);
     if (s->zero0) (void)hipFree(s->zero0);
     s->n0 = n;
     s->nz0 = int(zeros.size());
-    s->inv0 = dmalloc<double>(inv.size());
+    s->inv0 = dinv;
     s->cells0 = dmalloc<int32_t>(cells.size());
     s->zero0 = dmalloc<int32_t>(zeros.size());
     if (n) {
-        HIPCHK(hipMemcpy(s->inv0, inv.data(), inv.size() * sizeof(double), hipMemcpyHostToDevice));
         HIPCHK(hipMemcpy(s->cells0, cells.data(), cells.size() * sizeof(int32_t), hipMemcpyHostToDevice));
     }
     if (!zeros.empty()) HIPCHK(hipMemcpy(s->zero0, zeros.data(), zeros.size() * sizeof(int32_t), hipMemcpyHostToDevice));

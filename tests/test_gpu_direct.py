@@ -1,0 +1,91 @@
+"""The FP64 direct solve of level 0: its inverse is made on the device for symmetric positive definite systems (sizes off
+the elimination's blocks among them) and on the host otherwise; both solve the level-0 system."""
+import numpy as np
+import pytest
+
+import cirrus_amg as P
+import helpers as H
+
+pytestmark = pytest.mark.gpu
+
+
+def _grid(case):
+    """a single-level grid of one tile (so that a cycle is the direct solve), its types and operator"""
+    g = P.HADeviceGrid(log2_hash=(4,))
+    g.setTileHost(0, (0, 0, 0), P.LEAF)
+    g.rebuild()
+    g.finalize()
+    rng = np.random.default_rng(5)
+    types = np.full((1, 512), P.INTERIOR, np.uint8)
+    if case == "ragged":       # 512 - 75 unknowns: not a multiple of 32
+        types[0, rng.choice(512, 75, replace=False)] = P.DIRICHLET
+    if case == "few":          # a few unknowns only
+        types[:] = P.DIRICHLET
+        types[0, rng.choice(512, 20, replace=False)] = P.INTERIOR
+    g.set_cell_types(types)
+    g.prepare_types_and_coeffs(H.C0, H.R_MATRIX)
+    return g
+
+
+def _matrix(g):
+    """the level-0 system from the grid's types and coefficients"""
+    C = [g.channel(H.C0 + a)[0].astype(np.float64) for a in range(4)]
+    inside = g.cell_types()[0] == P.INTERIOR
+    cells = np.where(inside)[0]
+    uid = {c: i for i, c in enumerate(cells)}
+    A = np.zeros((len(cells), len(cells)))
+    for i, c in enumerate(cells):
+        l = [c >> 6, (c >> 3) & 7, c & 7]
+        A[i, i] = C[3][c]
+        for a, step in enumerate((64, 8, 1)):
+            if l[a] > 0 and c - step in uid:
+                A[i, uid[c - step]] += C[a][c]
+            if l[a] < 7 and c + step in uid:
+                A[i, uid[c + step]] += C[a][c + step]
+    return cells, A
+
+
+@pytest.mark.parametrize("case", ["full", "ragged", "few", "unsymmetric", "indefinite"])
+def test_level0_direct_solve(case):
+    g = _grid(case)
+    if case in ("unsymmetric", "indefinite"):
+        # a diagonal of its own for some cells: still diagonally dominant, no longer definite when negative;
+        # a face coefficient seen from one side only cannot be made here, so the unsymmetric form drops a
+        # diagonal, which leaves that cell's row empty and the system singular
+        d = g.channel(H.C0 + 3)
+        d[0, 77] = 0.0 if case == "unsymmetric" else -8.0
+        g.set_channel(H.C0 + 3, d)
+    cells, A = _matrix(g)
+    b = H.random_fill(1, 9)
+    g.set_channel(1, b)
+    o = P.default_opts(cycle=P.CYCLE_FAS_V, smoother=P.SMOOTH_JACOBI, coarsest_direct=1)
+    s = P.AMGSolver(g, H.C0, H.R_MATRIX, 1.0, 1.0)
+    if case == "unsymmetric":
+        with pytest.raises(P.CmgError) as e:
+            s.cycle(o, 4, 1, 3)
+        assert "singular" in str(e.value)
+        return
+    s.cycle(o, 4, 1, 3)
+    x = np.linalg.solve(A, b[0, cells].astype(np.float64))
+    z = g.channel(4)[0]
+    # the FP32 result of an FP64 solve: half an ulp, and the FP64 error of a condition number below 1e4
+    assert np.abs(z[cells] - x).max() <= 2.0**-24 * np.abs(x).max() * 1.01
+    rest = np.setdiff1d(np.arange(512), cells)
+    assert not z[rest].any()
+
+
+def test_pure_neumann_solve():
+    """an all-Neumann box: the level-0 system is the singular one with its constant part shifted"""
+    _, gp = H.build_pair("uniform2")
+    co = gp.tiles()[1]
+    types = gp.cell_types()
+    v = np.arange(512)
+    for t in np.where(gp.tiles()[2] == 1)[0]:
+        at = co[t] * 8 + np.stack([v >> 6, (v >> 3) & 7, v & 7], 1)
+        types[t, ((at == 0) | (at == 31)).any(1)] = P.NEUMANN
+    gp.set_cell_types(types)
+    gp.prepare_types_and_coeffs(H.C0, H.R_MATRIX)
+    gp.rhs_uniform(1, 3, True)
+    o = P.default_opts(cycle=P.CYCLE_FAS_V, smoother=P.SMOOTH_JACOBI, omega=2.0 / 3.0, coarsest_direct=1)
+    it, rel = P.AMGSolver(gp, H.C0, H.R_MATRIX, 1.0, 1.0).solve(relative_tolerance=1e-6, is_pure_neumann=True, opts=o)
+    assert rel < 1e-6 and it < 40
