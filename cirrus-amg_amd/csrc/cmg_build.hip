@@ -706,6 +706,7 @@ public:
                 s.used = true;
                 s.refine = ((rec[j].w >> 4) & 1) != 0;
             }
+            topo_.any_[l] = true;
         }
         topo_.max_level_ = max_level_;
         topo_.finalized_ = false;
@@ -762,8 +763,8 @@ public:
         read_back();
         T.level_start = start;
         for (int l = 0; l < L_; ++l) {
-            T.slot_tile_[l].assign(T.table_[l].size(), -1);
-            for (int t = start[l]; t < start[l + 1]; ++t) T.slot_tile_[l][T.t_slot[t]] = t;
+            T.slot_tile_[l] = ZeroArray<int32_t>(T.table_[l].size());
+            for (int t = start[l]; t < start[l + 1]; ++t) T.slot_tile_[l][T.t_slot[t]] = t + 1;
         }
         T.finalized_ = true;
     }

@@ -9,8 +9,11 @@
 
 #include <array>
 #include <cstdint>
+#include <cstdlib>
 #include <functional>
+#include <new>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "cirrus_amg.h"
@@ -31,12 +34,41 @@ using Coord = std::array<int32_t, 3>;
 
 inline int cell_index(int i, int j, int k) { return (i << 6) | (j << 3) | k; }
 
-// one hash slot of a level table: the tile identity plus its refine status
+// one hash slot of a level table: the tile identity plus its refine status (all bytes 0: free)
 struct Slot {
     Coord c{0, 0, 0};
     uint8_t type = 0;
     bool used = false;
     bool refine = false;   // REFINE_FLAG of mStatus
+};
+
+// a fixed-size array of zero bytes whose pages are touched on first use (a level's hash table
+// is sized for its finest use, 16 MB at 2^20 slots, and most of it is never touched)
+template <typename T>
+class ZeroArray {
+public:
+    ZeroArray() = default;
+    explicit ZeroArray(size_t n) : n_(n), p_(n ? static_cast<T*>(std::calloc(n, sizeof(T))) : nullptr)
+    {
+        if (n && !p_) throw std::bad_alloc();
+    }
+    ZeroArray(ZeroArray&& o) noexcept : n_(o.n_), p_(o.p_) { o.n_ = 0, o.p_ = nullptr; }
+    ZeroArray& operator=(ZeroArray&& o) noexcept
+    {
+        std::swap(n_, o.n_);
+        std::swap(p_, o.p_);
+        return *this;
+    }
+    ZeroArray(const ZeroArray&) = delete;
+    ZeroArray& operator=(const ZeroArray&) = delete;
+    ~ZeroArray() { std::free(p_); }
+    size_t size() const { return n_; }
+    T& operator[](size_t i) { return p_[i]; }
+    const T& operator[](size_t i) const { return p_[i]; }
+
+private:
+    size_t n_ = 0;
+    T* p_ = nullptr;
 };
 
 class Topology {
@@ -82,10 +114,11 @@ private:
     int max_level_ = -1;
     bool finalized_ = false;
     std::array<uint32_t, kMaxLevels> log2_{};
-    std::array<std::vector<Slot>, kMaxLevels> table_;
+    std::array<ZeroArray<Slot>, kMaxLevels> table_;
+    std::array<bool, kMaxLevels> any_{};   // the level's table has a used slot
     std::array<std::vector<int32_t>, kMaxLevels> compressed_;   // slot indices in slot order
     std::array<std::vector<int32_t>, kMaxLevels> touched_;      // slots claimed since the last compression
-    std::array<std::vector<int32_t>, kMaxLevels> slot_tile_;    // slot -> tile index
+    std::array<ZeroArray<int32_t>, kMaxLevels> slot_tile_;      // slot -> tile index + 1, 0 for none
 };
 
 // analytic SDFs shared by targets and assembly (float, no contraction)

@@ -26,7 +26,7 @@ Topology::Topology(float h0, int num_levels, const uint32_t* log2_hash) : h0_(h0
     for (int l = 0; l < num_levels; ++l) {
         if (log2_hash[l] < 1 || log2_hash[l] > 26) throw std::invalid_argument("log2 hash size out of range");
         log2_[l] = log2_hash[l];
-        table_[l].assign(size_t(1) << log2_hash[l], Slot{});
+        table_[l] = ZeroArray<Slot>(size_t(1) << log2_hash[l]);
     }
 }
 
@@ -73,6 +73,7 @@ int Topology::set_tile(int level, const Coord& c, uint8_t type)
     Slot& s = table_[level][k];
     if (!s.used) {
         s.used = true;
+        any_[level] = true;
         s.c = c;
         s.refine = false;
         touched_[level].push_back(int32_t(k));
@@ -89,6 +90,7 @@ void Topology::compress()
         touched_[l].clear();
         auto& out = compressed_[l];
         out.clear();
+        if (!any_[l]) continue;
         for (size_t k = 0; k < table_[l].size(); ++k)
             if (table_[l][k].used) out.push_back(int32_t(k));
         if (!out.empty()) max_level_ = l;
@@ -176,7 +178,7 @@ int Topology::tile_at(int level, const Coord& c) const
     if (level < 0 || level >= num_levels_) return -1;
     int k = probe(level, c);
     if (k < 0 || !table_[level][k].used) return -1;
-    return slot_tile_[level][k];
+    return slot_tile_[level][k] - 1;
 }
 
 void Topology::finalize()
@@ -186,9 +188,9 @@ void Topology::finalize()
     level_start.assign(num_levels_ + 1, 0);
     for (int l = 0; l < num_levels_; ++l) {
         level_start[l] = int32_t(t_level.size());
-        slot_tile_[l].assign(table_[l].size(), -1);
+        slot_tile_[l] = ZeroArray<int32_t>(table_[l].size());
         for (int32_t k : compressed_[l]) {
-            slot_tile_[l][k] = int32_t(t_level.size());
+            slot_tile_[l][k] = int32_t(t_level.size()) + 1;
             t_level.push_back(l);
             t_slot.push_back(k);
             t_coord.push_back(table_[l][k].c);
