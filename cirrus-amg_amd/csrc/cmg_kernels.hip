@@ -147,76 +147,6 @@ __device__ __forceinline__ float coef_q(const uint16_t* q, size_t i, float h)
     return float(__builtin_bit_cast(_Float16, q[i])) * h;
 }
 
-// element s (0..5, thread-varying) of (a.x, a.y, a.z, a.w, b.x, b.y) by selects,
-// with no private array (which the compiler would place in LDS)
-__device__ __forceinline__ int pick6(int4 a, int4 b, int s)
-{
-    int r = a.x;
-    r = s == 1 ? a.y : r;
-    r = s == 2 ? a.z : r;
-    r = s == 3 ? a.w : r;
-    r = s == 4 ? b.x : r;
-    r = s == 5 ? b.y : r;
-    return r;
-}
-
-// element s (0..7, thread-varying) of (a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w) by selects
-__device__ __forceinline__ int pick8(int4 a, int4 b, int s)
-{
-    int r = pick6(a, b, s);
-    r = s == 6 ? b.z : r;
-    r = s == 7 ? b.w : r;
-    return r;
-}
-
-// A one-tile stencil workgroup's record (launch-list order, 7 x 16 bytes, read with
-// scalar loads right after the launch): the tile, its level, type | octant << 8 and
-// parent; its halo record (face neighbours, their tile types packed in bytes, own
-// type in byte 7.3); the parents of the face neighbours and their octants (the
-// operator's fresh GHOST values, the cycle's pulled prolongation); its children by
-// octant (for a sweep that prolongs into them).  One round trip gives the workgroup every address it needs:
-// the tile's own loads and its halo loads follow at once.
-struct TileRec {
-    int t, level, meta, parent;
-    int4 ha, hb, ga, gb;
-    int4 ca, cb;   // children by octant (CHILD records only)
-    int tid;       // the thread's index among the threads working on the tile
-};
-
-// t = -1: padding entry, -2: the solve has stopped.  S is never null here (launches
-// outside a solve pass the grid's idle block, whose flag is never set), so the stop
-// flag is read with no branch and its load overlaps the record's.
-template <bool FRESH, bool STOP = true, bool CHILD = false>
-__device__ __forceinline__ TileRec rec_tile(const int4* __restrict__ rec, const double* __restrict__ S)
-{
-    const int4* r = rec + kRecWords * size_t(blockIdx.x);
-    const int4 r0 = r[0];
-    TileRec x;
-    x.ha = r[1];
-    x.hb = r[2];
-    if (FRESH) {
-        x.ga = r[3];
-        x.gb = r[4];
-    } else {
-        x.ga = make_int4(-1, -1, -1, -1);
-        x.gb = make_int4(-1, -1, 0, 0);
-    }
-    if (CHILD) {
-        x.ca = r[5];
-        x.cb = r[6];
-    } else {
-        x.ca = x.cb = make_int4(-1, -1, -1, -1);
-    }
-    x.t = (STOP && S[S_DONE] != 0.0) ? -2 : r0.x;
-    x.tid = threadIdx.x;
-    x.level = r0.y;
-    x.meta = r0.z;
-    x.parent = r0.w;
-    return x;
-}
-
-__device__ __forceinline__ float rec_h(const TopoView& tp, const TileRec& r) { return tp.h0 / float(1 << r.level); }
-
 // LoadAMGLaplacianTileData (src/AMGSolver.cu:395-543).
 // FRESH: the halo is evaluated the way AMGFullNegativeLaplacianOnLeafs sees it
 //   after PropagateToChildren + AccumulateToParentsOneStep: a GHOST cell is its

@@ -125,6 +125,13 @@ void launch_geo_apply(const DevGrid& d, int mode, const LaunchList& l, int subtr
 void launch_geo_gs(const DevGrid& d, int mode, int level, float* X, const float* B, int color, const double* S, hipStream_t st);
 void launch_geo_restrict(const DevGrid& d, int mode, int level, const float* X, float* B, float one_over_alpha,
                          const double* S, hipStream_t st);
+// a V-cycle's visit to a complete level (DevGrid::dense; 1 or 2 iterations) in two launches: post
+// false the iterations from x = 0, residual and restriction (x into T), post true the
+// prolongation and the iterations (x from T into X)
+void launch_geo_dense(const DevGrid& d, int mode, int level, bool post, int iters, float* X, float* T, float* B,
+                      float one_over_alpha, float P, const double* S, hipStream_t st);
+// a level 0 of one tile alone (DevGrid::root_alone): `iters` iterations from red, `iters` from black
+void launch_geo_root(const DevGrid& d, int mode, int iters, float* X, const float* B, const double* S, hipStream_t st);
 void launch_accumulate_ghosts_add(const DevGrid& d, float* Y, float coeff, const double* S, hipStream_t st);
 void launch_residual_interior(const DevGrid& d, const float* B, float* AX, hipStream_t st);
 void launch_djacobi_update(const DevGrid& d, float* X, const float* R, const float* D, float omega, hipStream_t st);

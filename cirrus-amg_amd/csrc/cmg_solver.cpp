@@ -1185,13 +1185,27 @@ void geo_vcycle(cmg_solver* s, const cmg_solve_opts* o, float* X, const float* F
     hipStream_t st = d.stream;
     const int mode = geo_mode(s);
     launch_nonfas_init(d, X, F, B, S, st);
+    // complete levels: all of a tile's passes in one launch
+    auto dense = [&](int l) { return d.dense[l] && o->level_iters >= 1 && o->level_iters <= 2 && fuse_rz_allowed(); };
     for (int l = d.max_level; l > 0; --l) {
+        if (dense(l)) {
+            launch_geo_dense(d, mode, l, false, o->level_iters, X, s->tmp, B, s->Rr, s->P, S, st);
+            continue;
+        }
         geo_gauss_seidel(s, o->level_iters, 0, l, X, B, S);
         launch_geo_restrict(d, mode, l, X, B, s->Rr, S, st);
     }
-    geo_gauss_seidel(s, o->coarsest_iters / 2, 0, 0, X, B, S);
-    geo_gauss_seidel(s, o->coarsest_iters / 2, 1, 0, X, B, S);
+    if (coarsest_iterate_available(d)) {
+        launch_geo_root(d, mode, o->coarsest_iters / 2, X, B, S, st);
+    } else {
+        geo_gauss_seidel(s, o->coarsest_iters / 2, 0, 0, X, B, S);
+        geo_gauss_seidel(s, o->coarsest_iters / 2, 1, 0, X, B, S);
+    }
     for (int l = 1; l <= d.max_level; ++l) {
+        if (dense(l)) {
+            launch_geo_dense(d, mode, l, true, o->level_iters, X, s->tmp, B, s->Rr, s->P, S, st);
+            continue;
+        }
         // GMG prolongs into LEAF|NONLEAF|GHOST tiles, CMG into LEAF|NONLEAF only
         launch_prolong_add(d, l, X, s->P, S, st, mode == 1);
         geo_gauss_seidel(s, o->level_iters, 1, l, X, B, S);
