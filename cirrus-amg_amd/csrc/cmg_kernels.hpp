@@ -167,12 +167,18 @@ int launch_net_train(const float* X, const float* E, const int32_t* idx, int n, 
                      double* lpart, int max_wg, bool bf16, hipStream_t st);
 void launch_net_reduce(const float* gpart, const double* lpart, int nwg, int n, float* grad, double* loss, hipStream_t st);
 void launch_adam(float* W, float* M, float* V, const float* G, int t, float lr, float b1, float b2, float eps, hipStream_t st);
+// layer 2's weights as launch_net_infer reads them, into P (infer_pack_floats())
+size_t infer_pack_floats();
+void launch_infer_pack(const float* W, float* P, hipStream_t st);
+// W: the weights followed by launch_infer_pack's
 void launch_net_infer(const DevGrid& d, const LaunchList& l, const float* R, const float* D, const float* W, float* Y,
                       const double* S, hipStream_t st);
 void launch_mfma_probe(int K, const uint16_t* A, const uint16_t* B, float* C, hipStream_t st);
 // learned pre-smoothing acceptance on the finest level: keep the net's correction
 // (in Y) on a tile when it lowers the tile's residual, else the first Jacobi sweep
-// count (optional): [0] += tiles judged, [1] += tiles that kept the net's correction
+// count (optional): kLearnedSlots pairs, kLearnedStride words apart, whose sums are the tiles judged
+// and the tiles that kept the net's correction
+constexpr int kLearnedSlots = 64, kLearnedStride = 32;
 void launch_learned_accept(const DevGrid& d, int level, const float* Y, float* X, Coef C, const float* B, float w,
                            const double* S, hipStream_t st, unsigned int* count = nullptr);
 

@@ -52,9 +52,14 @@ __device__ __forceinline__ int tap_off(int t, int E) { return (t / 9 - 1) * E * 
 
 __device__ __forceinline__ uint16_t bf16_bits(float f) { return uint16_t(__float_as_uint(bf16_round(f)) >> 16); }
 
+// (one instruction; NaN gives 0)
+__device__ __forceinline__ float relu(float x) { return __builtin_amdgcn_fmed3f(x, 0.0f, INFINITY); }
+
 __device__ __forceinline__ uint32_t pack_relu_bf16(float lo, float hi)
 {
-    return uint32_t(bf16_bits(lo > 0 ? lo : 0.0f)) | (uint32_t(bf16_bits(hi > 0 ? hi : 0.0f)) << 16);
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    typedef __bf16 b16x2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{relu(lo), relu(hi)}, b16x2));
 }
 
 // ---------------------------------------------------------------- gather ----
@@ -581,34 +586,43 @@ __global__ __launch_bounds__(256) void adam(float* __restrict__ W, float* __rest
 
 // -------------------------------------------------------------- inference ----
 // BF16 MFMA forward pass on the tile's own 8^3 cells: y = net(x), x gathered
-// from channel R / D as for training.  Persistent: each 256-thread workgroup
-// (4 wave64s) holds the weights in registers and walks the tiles of a list.
-// All three layers run on v_mfma_f32_16x16x{32,16}_bf16 with output channels
-// (or taps) as the M side and 16 positions of the 10^3 volume as the N side:
-//   layer 1: [16 co x 32 (27 taps + 5 zero)] x [32 x 16 positions]
-//   layer 2: per tap pair, [16 co x 32 (2 taps x 16 ci)] x [32 x 16 positions]
-//            (14 pairs, the 28th tap zero)
-//   layer 3: U[tap][q] = sum_ci W3[ci][tap] a2[q][ci] for 9 taps at a time
-//            ([16 (9 used) x 16 ci] x [16 x 16 positions]), then
-//            y[p] = sum over taps of U[tap][p + off(tap)] in a fixed order.
+// from channel R / D as for training.  Persistent: each 512-thread workgroup
+// (8 wave64s) walks the tiles of a list.
+// All three layers run on v_mfma_f32_16x16x32_bf16 with output channels as the M side and 16
+// positions as the N side:
+//   layer 1: [16 co x 32 (27 taps + 5 zero)] x [32 x 16 positions of the 10^3 volume]
+//   layers 2 and 3: per pair of the nine taps in a plane, [16 rows x 32 (2 taps x 16 ci)] x [32 x
+//            16 positions of one plane], 5 pairs (the tenth tap zero).  In layer 2 an operand of plane
+//            i serves the outputs of planes i - 1, i and i + 1 with the weights of three taps across
+//            the planes: 50 operands and 140 products for the ten planes of a column of positions.
+//            Layer 3 has one output channel, so its rows are the three taps across the planes and
+//            output i adds row 0 of plane i - 1, row 1 of plane i and row 2 of plane i + 1; it runs
+//            on the tile's own 8^3 cells.
 // Activations are rounded to bfloat16 after each ReLU, products accumulate in
 // FP32 (the same rounding points as the training forward pass in BF16 mode).
-// The input of the next tile (r / D on 512 own and 384 face-halo cells, 3.5
+// The input of the next tile (r / D on 512 own and 384 face-halo cells, 1.75
 // cells per thread) is loaded into registers while the current tile's layer 3
 // is computed; the neighbours come from the tile's 32-byte halo record.
-// LDS (71,488 B, two workgroups per CU).  Activations are stored by channel
-// group so that the 16 positions one MFMA operand reads are contiguous (no bank
-// conflicts): a1 as [2 halves of 8 ch][1000 positions][8 ch], a2 as
-// [4 quarters of 4 ch][1000 positions][4 ch].
-//   [0, 32000)        a1, bf16                         | U[9][1000] fp32
-//   [0, 36000)                                          | (aliases a1)
-//   [36000, 36032)    zero bytes (out-of-volume taps of layer 2)
-//   [36032, 68032)    a2, bf16
-//   [68032, 71488)    x on the zero-padded 12^3 volume, bf16 (edges and
-//                     corners of the 10^3 volume and the padding stay 0)
-
-constexpr int IL_A1 = 0, IL_ZERO = 36000, IL_A2 = 36032, IL_X = 68032, IL_BYTES = 71488;
-constexpr int IN_PT = 4;   // input cells per thread (896 = 512 own + 384 halo, 256 threads)
+// What bounds it is the issue of vector instructions (26.4 million a call on 3,680 tiles, 44 us of
+// it), the LDS reads (27 million cycles of 256 CUs, 44 us) and the matrix cores (36 us), which
+// overlap in part, and a last round of tiles that is not full.  Operands one tap pair at a time
+// cost 1,330 reads of 1 KB a tile (630 now) and, without the zeros around a1, a test of the tap's
+// place for each.  3,680 tiles of sphere-256: 217 -> 82 us (256 threads a workgroup, one block of
+// positions after another: 217; tap pairs outermost, weights loaded once for 16 blocks: 174; 512
+// threads, so four waves a SIMD: 141; zeros around a1: 113).
+// LDS (81,648 B, two workgroups per CU).  Activations are stored by channel half so that the 16
+// positions one MFMA operand reads are contiguous but for the holes (few bank conflicts):
+//   [0, 44912)        a1, bf16 [2 halves of 8 ch][positions][8 ch].  Rows and planes of 10 are 11
+//                     apart and 133 places lie before, between and after the halves: whatever a
+//                     tap reads outside the volume is one of these zeros
+//   [44912, 77232)    a2, bf16 [2 halves of 8 ch][10 planes][100 positions and a zero][8 ch]
+//   [77232, 80688)    x on the zero-padded 12^3 volume, bf16 (edges and corners of the 10^3
+//                     volume and the padding stay 0)
+//   [80688, 81648)    layer 3's weights, bf16 [5 pairs][2 taps][2 halves of 8 ci][3 planes][8 ci]
+constexpr int IL_A1 = 0, IL_A2 = 44912, IL_X = 77232, IL_W3 = 80688, IL_BYTES = 81648;
+constexpr int IL_HALF = 1343 * 16;   // from a1's lower channels to its upper ones
+__device__ __forceinline__ int a1_place(int i, int j, int k) { return IL_A1 + (133 + (i * 11 + j) * 11 + k) * 16; }
+constexpr int IN_PT = 2;   // input cells per thread (896 = 512 own + 384 halo, 512 threads)
 
 // registers of one tile's input: padded-volume position (-1: none), r, D, cell type
 struct InferIn {
@@ -628,13 +642,15 @@ __device__ __forceinline__ void infer_issue(InferIn& in, const TopoView& tp, int
         in.ct[m] = 0;
     }
     if (t < 0) return;
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));   // (places kept over the tiles would spill)
     const int4* hr = reinterpret_cast<const int4*>(tp.halo + size_t(t) * 8);
     const int4 ha = hr[0], hb = hr[1];
     const int nb[6] = {ha.x, ha.y, ha.z, ha.w, hb.x, hb.y};
     const uint32_t ty03 = uint32_t(hb.z), ty45 = uint32_t(hb.w);
 #pragma unroll
     for (int m = 0; m < IN_PT; ++m) {
-        const int e = threadIdx.x + 256 * m;
+        const int e = tid + 512 * m;
         if (e >= 896) continue;
         int tt, l0, l1, l2, p0, p1, p2;   // source tile, its cell, padded position
         if (e < 512) {
@@ -668,7 +684,7 @@ __device__ __forceinline__ void infer_issue(InferIn& in, const TopoView& tp, int
     }
 }
 
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void net_infer(TopoView tp, const int32_t* __restrict__ tiles, int n,
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void net_infer(TopoView tp, const int32_t* __restrict__ tiles, int n,
                                                  const float* __restrict__ R, const float* __restrict__ D,
                                                  const float* __restrict__ W, float* __restrict__ Y,
                                                  const double* __restrict__ S)
@@ -684,32 +700,27 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void n
         const int tap = 8 * grp + j;
         w1v[j] = tap < 27 ? short(bf16_bits(W[col * 27 + tap])) : short(0);
     }
-    // layer 2, pair m: tap 2m + (grp >> 1), input channel 8 (grp & 1) + j
-    s16x8 w2v[14];
-#pragma unroll
-    for (int m = 0; m < 14; ++m) {
-        const int tap = 2 * m + (grp >> 1);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const int ci = 8 * (grp & 1) + j;
-            w2v[m][j] = tap < 27 ? short(bf16_bits(W[OW2 + (col * NC + ci) * 27 + tap])) : short(0);
-        }
-    }
-    // layer 3, group g: row = tap g*9 + col (col < 9), k = input channel 4 grp + j
-    bf16x4 w3v[3];
-#pragma unroll
-    for (int g = 0; g < 3; ++g)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-            w3v[g][j] = col < 9 ? short(bf16_bits(W[OW3 + (4 * grp + j) * 27 + g * 9 + col])) : short(0);
     // layer-1 tap offsets on the padded 12^3 volume (taps 27..31 are zero taps)
     int o1[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) o1[j] = 8 * grp + j < 27 ? tap_off(8 * grp + j, 12) : 0;
-    if (tid < 8) reinterpret_cast<uint32_t*>(lds + IL_ZERO)[tid] = 0u;
-    for (int e = tid; e < 1728 / 2; e += 256) reinterpret_cast<uint32_t*>(lds + IL_X)[e] = 0u;
+    for (int e = tid; e < IL_X / 16; e += 512) reinterpret_cast<uint4*>(lds)[e] = make_uint4(0u, 0u, 0u, 0u);
+    for (int e = tid; e < 1728 / 2; e += 512) reinterpret_cast<uint32_t*>(lds + IL_X)[e] = 0u;
+    if (tid < 480) {
+        const int j = tid & 7, d = (tid >> 3) % 3, g = (tid / 24) & 3, r = 2 * (tid / 96) + (g >> 1);
+        reinterpret_cast<uint16_t*>(lds + IL_W3)[tid] = r < 9 ? bf16_bits(W[OW3 + (8 * (g & 1) + j) * 27 + 9 * d + r]) : uint16_t(0);
+    }
     const uint16_t* xs = reinterpret_cast<const uint16_t*>(lds + IL_X);
-    float* U = reinterpret_cast<float*>(lds);
+    // per block of 16 positions of this wave (block wave + 8 b; the last ones lie beyond the volume:
+    // computed like its last position and dropped) the places in x and in a1
+    int place[8];   // of 2 bytes in x + 2048 times that of 16 in a1
+#pragma unroll
+    for (int b = 0; b < 8; ++b) {
+        const int p = min(16 * (wave + 8 * b) + col, NV - 1), i = p / 100, j = (p / 10) % 10, kk = p % 10;
+        place[b] = ((i + 1) * 12 + j + 1) * 12 + kk + 1 + a1_place(i, j, kk) / 16 * 2048;
+    }
+    // of layer 2's positions 16 wave + col of a plane, in the first plane
+    const int p2 = min(16 * wave + col, 99), plane2 = a1_place(0, p2 / 10, p2 % 10);
 
     InferIn cur;
     infer_issue(cur, tp, blockIdx.x < n ? tiles[blockIdx.x] : -1, R, D);
@@ -730,103 +741,110 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void n
             infer_issue(cur, tp, bn < n ? tiles[bn] : -1, R, D);
             continue;
         }
-        // layer 1
-        for (int mb = wave; mb < NBLK; mb += 4) {
-            const int p = mb * 16 + col;
-            const bool ok = p < NV;
-            const int pc = ok ? p : 0;
-            const int c12 = ((pc / 100 + 1) * 12 + (pc / 10) % 10 + 1) * 12 + pc % 10 + 1;
-            s16x8 xv;
+        // (an address for every block and operand, kept over the tiles, would spill)
 #pragma unroll
-            for (int j = 0; j < 8; ++j) xv[j] = (ok && 8 * grp + j < 27) ? short(xs[c12 + o1[j]]) : short(0);
+        for (int j = 0; j < 8; ++j) asm volatile("" : "+v"(o1[j]));
+        int grp = lane >> 4;
+        asm volatile("" : "+v"(grp));
+        // layer 1 (taps 24, 25, 26 and zeros for the last lanes)
+        const uint32_t m1[4] = {~0u, grp == 3 ? 0xffffu : ~0u, grp == 3 ? 0u : ~0u, grp == 3 ? 0u : ~0u};
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            const int p = 16 * (wave + 8 * q) + col;
+            const bool ok = p < NV;
+            const int c12 = place[q] & 2047, c11 = (place[q] >> 11) * 16;
+            uint32_t xw[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) xw[j] = (uint32_t(xs[c12 + o1[2 * j]]) | uint32_t(xs[c12 + o1[2 * j + 1]]) << 16) & m1[j];
+            const s16x8 xv = __builtin_bit_cast(s16x8, make_uint4(xw[0], xw[1], xw[2], xw[3]));
             f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
             acc = mfma32(w1v, xv, acc);
             if (ok) {
                 uint2 v;
                 v.x = pack_relu_bf16(acc[0], acc[1]);
                 v.y = pack_relu_bf16(acc[2], acc[3]);
-                *reinterpret_cast<uint2*>(lds + IL_A1 + (grp >> 1) * 16000 + p * 16 + (grp & 1) * 8) = v;
+                *reinterpret_cast<uint2*>(lds + c11 + (grp >> 1) * IL_HALF + (grp & 1) * 8) = v;
             }
         }
         __syncthreads();
-        // layer 2: two position blocks per step (independent accumulators), the
-        // next tap pair's operands read from LDS while this pair's MFMAs run
-        for (int mb = wave; mb < NBLK; mb += 8) {
-            const int p0 = mb * 16 + col, p1 = p0 + 64;
-            const bool ok0 = p0 < NV, ok1 = p1 < NV;
-            const int pi0 = p0 / 100, pj0 = (p0 / 10) % 10, pk0 = p0 % 10;
-            const int pi1 = p1 / 100, pj1 = (p1 / 10) % 10, pk1 = p1 % 10;
-            auto operand = [&](int m, int p, bool ok, int pi, int pj, int pk) {
-                const int tap = 2 * m + (grp >> 1);
-                const int di = tap / 9 - 1, dj = (tap / 3) % 3 - 1, dk = tap % 3 - 1;
-                const bool in = ok && tap < 27 && unsigned(pi + di) < 10u && unsigned(pj + dj) < 10u && unsigned(pk + dk) < 10u;
-                const int addr = in ? IL_A1 + (grp & 1) * 16000 + (p + di * 100 + dj * 10 + dk) * 16 : IL_ZERO;
-                return *reinterpret_cast<const s16x8*>(lds + addr);
-            };
-            f32x4 acc0 = {0.0f, 0.0f, 0.0f, 0.0f}, acc1 = {0.0f, 0.0f, 0.0f, 0.0f};
-            s16x8 b0 = operand(0, p0, ok0, pi0, pj0, pk0), b1 = operand(0, p1, ok1, pi1, pj1, pk1);
+        // layer 2: wave w has positions 16 w .. of all ten planes
+        if (wave < 7) {
+            f32x4 acc[10];
 #pragma unroll
-            for (int m = 0; m < 14; ++m) {
-                s16x8 n0 = b0, n1 = b1;
-                if (m + 1 < 14) {
-                    n0 = operand(m + 1, p0, ok0, pi0, pj0, pk0);
-                    n1 = operand(m + 1, p1, ok1, pi1, pj1, pk1);
+            for (int i = 0; i < 10; ++i) acc[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            const uint4* wq = reinterpret_cast<const uint4*>(W + NW) + lane;   // (infer_pack)
+            uint4 w[3] = {wq[0], wq[64], wq[128]};
+#pragma unroll 1
+            for (int m = 0; m < 5; ++m) {
+                uint4 wn[3];
+#pragma unroll
+                for (int d = 0; d < 3; ++d) wn[d] = wq[64 * (3 * min(m + 1, 4) + d)];
+                const int r = 2 * m + (grp >> 1);   // (no tap 9: the hole at the end of a row)
+                const int at = (grp & 1) * IL_HALF + (r < 9 ? plane2 + ((r / 3 - 1) * 11 + r % 3 - 1) * 16 : a1_place(0, 0, 10));
+#pragma unroll
+                for (int i = 0; i < 10; ++i) {
+                    const s16x8 x = *reinterpret_cast<const s16x8*>(lds + at + 1936 * i);
+                    if (i > 0) acc[i - 1] = mfma32(__builtin_bit_cast(s16x8, w[2]), x, acc[i - 1]);
+                    acc[i] = mfma32(__builtin_bit_cast(s16x8, w[1]), x, acc[i]);
+                    if (i < 9) acc[i + 1] = mfma32(__builtin_bit_cast(s16x8, w[0]), x, acc[i + 1]);
                 }
-                acc0 = mfma32(w2v[m], b0, acc0);
-                acc1 = mfma32(w2v[m], b1, acc1);
-                b0 = n0;
-                b1 = n1;
+#pragma unroll
+                for (int d = 0; d < 3; ++d) w[d] = wn[d];
             }
-            if (ok0) {
-                uint2 v;
-                v.x = pack_relu_bf16(acc0[0], acc0[1]);
-                v.y = pack_relu_bf16(acc0[2], acc0[3]);
-                *reinterpret_cast<uint2*>(lds + IL_A2 + grp * 8000 + p0 * 8) = v;
-            }
-            if (ok1) {
-                uint2 v;
-                v.x = pack_relu_bf16(acc1[0], acc1[1]);
-                v.y = pack_relu_bf16(acc1[2], acc1[3]);
-                *reinterpret_cast<uint2*>(lds + IL_A2 + grp * 8000 + p1 * 8) = v;
+            const int p = 16 * wave + col;
+            if (p < 100) {
+#pragma unroll
+                for (int i = 0; i < 10; ++i) {
+                    uint2 v;
+                    v.x = pack_relu_bf16(acc[i][0], acc[i][1]);
+                    v.y = pack_relu_bf16(acc[i][2], acc[i][3]);
+                    *reinterpret_cast<uint2*>(lds + IL_A2 + (grp >> 1) * 16160 + (grp & 1) * 8 + p * 16 + 1616 * i) = v;
+                }
             }
         }
         __syncthreads();
         // the next tile's input loads fly while layer 3 runs (issued here, after
         // layer 2, whose register needs are the kernel's peak)
         infer_issue(cur, tp, bn < n ? tiles[bn] : -1, R, D);
-        // layer 3 in three groups of 9 taps (di = g - 1)
-        float y0 = 0.0f, y1 = 0.0f;
+        // layer 3 on the tile's cells: wave w has cells 16 (w & 3) .. of planes 4 (w >> 2) ..
+        {
+            f32x4 acc[6];
 #pragma unroll
-        for (int g = 0; g < 3; ++g) {
-            for (int mb = wave; mb < NBLK; mb += 4) {
-                const int p = mb * 16 + col;
-                const bool ok = p < NV;
-                bf16x4 av = {0, 0, 0, 0};
-                if (ok) av = *reinterpret_cast<const bf16x4*>(lds + IL_A2 + grp * 8000 + p * 8);
-                f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-                acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(w3v[g], av, acc, 0, 0, 0);
-                if (ok) {
+            for (int i = 0; i < 6; ++i) acc[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            const int c = wave & 3, h = wave >> 2;
+            // rows 0..2 hold the weights of the three planes
+            const unsigned char* w3 = lds + (col < 3 ? IL_W3 + (3 * grp + col) * 16 : IL_A1);
+            const int ws = col < 3 ? 192 : 0;
+            const int half = IL_A2 + (grp & 1) * 16160 + h * 6464;
+#pragma unroll 1
+            for (int m = 0; m < 5; ++m) {
+                const int r = 2 * m + (grp >> 1);   // (no tap 9: the hole at the end of a plane)
+                const int at = half + (r < 9 ? (2 * c + (col >> 3) + r / 3) * 160 + ((col & 7) + r % 3) * 16 : 1600);
+                const s16x8 w = *reinterpret_cast<const s16x8*>(w3 + ws * m);
 #pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        if (4 * grp + e < 9) U[(4 * grp + e) * NV + p] = acc[e];
+                for (int i = 0; i < 6; ++i) acc[i] = mfma32(w, *reinterpret_cast<const s16x8*>(lds + at + 1616 * i), acc[i]);
+            }
+            if (grp == 0) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const size_t cell = size_t(t) * 512 + 64 * (4 * h + q) + 16 * c + col;
+                    Y[cell] = (tp.ctype[cell] & INTERIOR) ? acc[q][0] + acc[q + 1][1] + acc[q + 2][2] : 0.0f;
                 }
             }
-            __syncthreads();
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const int v = tid + 256 * h;
-                const int q = ((v >> 6) + 1 + (g - 1)) * 100 + (((v >> 3) & 7) + 1) * 10 + (v & 7) + 1;
-                float acc = h ? y1 : y0;
-#pragma unroll
-                for (int s9 = 0; s9 < 9; ++s9) acc += U[s9 * NV + q + (s9 / 3 - 1) * 10 + (s9 % 3 - 1)];
-                if (h) y1 = acc; else y0 = acc;
-            }
-            __syncthreads();
         }
-        const size_t base = size_t(t) * 512;
-        Y[base + tid] = (tp.ctype[base + tid] & INTERIOR) ? y0 : 0.0f;
-        Y[base + tid + 256] = (tp.ctype[base + tid + 256] & INTERIOR) ? y1 : 0.0f;
     }
+}
+
+// the weights of layer 2 for net_infer, bf16: [5 pairs of in-plane taps][3 planes][64 lanes][8],
+// row lane & 15 = output channel, in-plane tap 2 m + lane / 32, input channel 8 (lane / 16 & 1) + j
+constexpr int IPACK = 15 * 512;
+__global__ __launch_bounds__(256) void infer_pack(const float* __restrict__ W, uint16_t* __restrict__ P)
+{
+    const int e = blockIdx.x * 256 + threadIdx.x;
+    if (e >= IPACK) return;
+    const int j = e & 7, lane = (e >> 3) & 63, d = (e >> 9) % 3, m = (e >> 9) / 3;
+    const int r = 2 * m + (lane >> 5), ci = 8 * ((lane >> 4) & 1) + j;
+    P[e] = r < 9 ? bf16_bits(W[OW2 + ((lane & 15) * NC + ci) * 27 + 9 * d + r]) : uint16_t(0);
 }
 
 // in-bounds check of the MFMA operand layouts: one wave64, C = A B for a
@@ -892,6 +910,13 @@ int launch_net_train(const float* X, const float* E, const int32_t* idx, int n, 
 
 size_t net_pack_floats() { return size_t(k::NPACK); }
 
+size_t infer_pack_floats() { return size_t(k::IPACK / 2); }
+
+void launch_infer_pack(const float* W, float* P, hipStream_t st)
+{
+    k::infer_pack<<<(k::IPACK + 255) / 256, 256, 0, st>>>(W, reinterpret_cast<uint16_t*>(P));
+}
+
 void launch_net_reduce(const float* gpart, const double* lpart, int nwg, int n, float* grad, double* loss, hipStream_t st)
 {
     k::net_reduce<<<(k::NW + 63) / 64, 64, 0, st>>>(gpart, lpart, nwg, n, grad, loss);
@@ -913,7 +938,7 @@ void launch_net_infer(const DevGrid& d, const LaunchList& l, const float* R, con
     (void)attr;
     // persistent: two workgroups per CU (68 KB of LDS each)
     const int grid = std::max(1, std::min(l.n, d.wg_cap / 4));
-    k::net_infer<<<grid, 256, k::IL_BYTES, st>>>(view(d), l.d, l.n, R, D, W, Y, S);
+    k::net_infer<<<grid, 512, k::IL_BYTES, st>>>(view(d), l.d, l.n, R, D, W, Y, S);
 }
 
 void launch_mfma_probe(int K, const uint16_t* A, const uint16_t* B, float* C, hipStream_t st)

@@ -38,8 +38,8 @@ struct cmg_solver {
     float* tmp = nullptr;          // Jacobi ping-pong buffer
     float* scratch = nullptr;      // cycle scratch of flexible CG (keeps Ap)
     float* dense_b = nullptr;      // FAS-saved right-hand sides of the complete levels (launch_dense_visit)
-    float* net_w = nullptr;        // learned tile smoother weights (7776 floats)
-    unsigned int* lcount = nullptr;   // learned steps of the last solve: tiles judged, tiles kept
+    float* net_w = nullptr;        // learned tile smoother weights (7776 floats), then launch_infer_pack's
+    unsigned int* lcount = nullptr;   // learned steps of the last solve (launch_learned_accept's counters)
     uint16_t* q16 = nullptr;          // FP16 copies of the four coefficient channels / h (cycle_coef_fp16)
     unsigned int* qbad = nullptr;     // workgroups whose FP16 copy has a value that does not fit
     // exact per-level codes of the face coefficients (Coef::w / lut): cell words, tables,
@@ -1846,7 +1846,7 @@ cmg_status solver_solve(cmg_solver* s, const cmg_solve_opts* o, cmg_solve_stats*
         ensure_buffers(s);
         const bool amg = s->family == CMG_SOLVER_AMG;
         if (amg) ensure_fp64(s);
-        if (o->learned) HIPCHK(hipMemset(s->lcount, 0, 2 * sizeof(unsigned int)));   // counts of this solve
+        if (o->learned) HIPCHK(hipMemset(s->lcount, 0, kLearnedSlots * kLearnedStride * sizeof(unsigned int)));   // counts of this solve
         if (amg && o->coarsest_direct) ensure_direct(s, o->is_pure_neumann != 0);
         if (amg && o->cycle_coef_fp16) prepare_coef_fp16(s);
         if (amg) prepare_coef_codes(s);
@@ -1990,12 +1990,14 @@ cmg_status solver_set_net(cmg_solver* s, const float* w)
 {
     if (!s || !w) return CMG_ERR_BAD_ARG;
     CMG_TRY({
-        if (!s->net_w) s->net_w = dmalloc<float>(kNetWeights);
+        if (!s->net_w) s->net_w = dmalloc<float>(kNetWeights + infer_pack_floats());
         if (!s->lcount) {
-            s->lcount = dmalloc<unsigned int>(2);
-            HIPCHK(hipMemset(s->lcount, 0, 2 * sizeof(unsigned int)));
+            s->lcount = dmalloc<unsigned int>(kLearnedSlots * kLearnedStride);
+            HIPCHK(hipMemset(s->lcount, 0, kLearnedSlots * kLearnedStride * sizeof(unsigned int)));
         }
         HIPCHK(hipMemcpy(s->net_w, w, kNetWeights * sizeof(float), hipMemcpyHostToDevice));
+        launch_infer_pack(s->net_w, s->net_w + kNetWeights, nullptr);
+        HIPCHK(hipStreamSynchronize(nullptr));
         if (s->gexec) (void)hipGraphExecDestroy(s->gexec), s->gexec = nullptr;   // the graph holds the old pointer
     });
     return CMG_OK;
@@ -2021,11 +2023,14 @@ cmg_status solver_learned_counts(cmg_solver* s, uint64_t* judged, uint64_t* kept
     if (!s || !judged || !kept) return CMG_ERR_BAD_ARG;
     if (!s->lcount) return CMG_ERR_STATE;
     CMG_TRY({
-        unsigned int h[2] = {0, 0};
+        std::vector<unsigned int> h(kLearnedSlots * kLearnedStride);
         HIPCHK(hipStreamSynchronize(s->g->dev.stream));
-        HIPCHK(hipMemcpy(h, s->lcount, sizeof(h), hipMemcpyDeviceToHost));
-        *judged = h[0];
-        *kept = h[1];
+        HIPCHK(hipMemcpy(h.data(), s->lcount, h.size() * sizeof(unsigned int), hipMemcpyDeviceToHost));
+        *judged = *kept = 0;
+        for (int i = 0; i < kLearnedSlots; ++i) {
+            *judged += h[i * kLearnedStride];
+            *kept += h[i * kLearnedStride + 1];
+        }
     });
     return CMG_OK;
 }
