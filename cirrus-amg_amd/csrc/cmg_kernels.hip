@@ -2448,12 +2448,15 @@ __global__ __launch_bounds__(512) void to_float(const int32_t* __restrict__ list
 // deterministic single-workgroup sum of partials, then the scalar step of the
 // PCG recurrence (alpha, convergence test, beta), replacing TernaryOnArray
 // one thread's share of a finish reduction: terms threadIdx.x, threadIdx.x + blockDim.x, ...
-// added in index order; U terms are loaded together (masked past n), so a thread's loads
-// overlap in one round trip per U terms
-template <int U, bool TWO>
+// added in index order; four terms are loaded together (masked past n).  What bounds it is the
+// chain load, sum, scalars, store of one workgroup; 40 terms at a time, most of them masked, and
+// the scalars loaded after the sum took 4.4 us a reduction on 512 tiles (2.9 now), 5.5 on 4,992
+// (4.5) and 8.7 on 35,712 (6.8)
+template <bool TWO>
 __device__ __forceinline__ void finish_terms(const double* __restrict__ p, const double* __restrict__ p2, int n, double& v,
                                              double& v2)
 {
+    constexpr int U = 4;
     const int step = blockDim.x;
     for (int i = threadIdx.x; i < n; i += U * step) {
         double a[U], b[U];
@@ -2473,51 +2476,57 @@ __device__ __forceinline__ void finish_terms(const double* __restrict__ p, const
     }
 }
 
-// thread 0 of finish (1024 threads): the 16 wave sums, in wave order, into the scalars of `kind`
-__device__ __forceinline__ void finish_apply(double* __restrict__ S, int kind, const double* red, const double* red2)
+// thread 0 of finish (1024 threads): the 16 wave sums, in wave order, into the scalars of `kind`;
+// v: the scalars as they stood.  Returns the stop code afterwards.
+__device__ __forceinline__ double finish_apply(double* __restrict__ S, const double* v, int kind, const double* red,
+                                               const double* red2)
 {
     double s = 0, s2 = 0;
-    for (int i = 0; i < 16; ++i) { s += red[i]; s2 += red2[i]; }
+    for (int i = 0; i < 16; ++i) s += red[i];
+    if (kind == FIN_MEAN || kind == FIN_BETA_FLEX)
+        for (int i = 0; i < 16; ++i) s2 += red2[i];
+    double done = v[S_DONE];
     switch (kind) {
-    case FIN_SUM: S[S_TMP] = s; break;
-    case FIN_GAMMA0: S[S_GAMMA] = s; break;
+    case FIN_SUM: S[S_TMP] = s; return done;
+    case FIN_GAMMA0: S[S_GAMMA] = s; return done;
+    case FIN_MEAN: S[S_MEAN] = s / s2; return done;
     case FIN_ALPHA:
         S[S_FP] = s;
-        if (!isfinite(s)) S[S_DONE] = 3;
-        else if (s == 0.0) S[S_DONE] = 2;
-        else S[S_ALPHA] = S[S_GAMMA] / s;
+        if (!isfinite(s)) done = 3;
+        else if (s == 0.0) done = 2;
+        else S[S_ALPHA] = v[S_GAMMA] / s;
         break;
-    case FIN_RR:
+    case FIN_RR: {
+        const double it = v[S_ITER] + 1;
         S[S_RR] = s;
-        S[S_ITER] += 1;
-        if (!isfinite(s)) S[S_DONE] = 3;
-        else if (S[S_STRIDE] > 0 && s < S[S_THR2] && fmod(S[S_ITER], S[S_STRIDE]) == 0.0) S[S_DONE] = 1;
-        else if (S[S_ITER] >= S[S_MAXIT]) S[S_DONE] = 4;
+        S[S_ITER] = it;
+        if (!isfinite(s)) done = 3;
+        else if (v[S_STRIDE] > 0 && s < v[S_THR2] && fmod(it, v[S_STRIDE]) == 0.0) done = 1;
+        else if (it >= v[S_MAXIT]) done = 4;
         break;
+    }
     case FIN_BETA:
-        S[S_GAMMA_OLD] = S[S_GAMMA];
+    case FIN_BETA_FLEX: {
+        // flexible CG (Polak-Ribiere): beta = z.(r - r_old) / gamma_old = -alpha z.Ap / gamma_old
+        const double beta = kind == FIN_BETA ? s / v[S_GAMMA] : -v[S_ALPHA] * s2 / v[S_GAMMA];
+        S[S_GAMMA_OLD] = v[S_GAMMA];
         S[S_GAMMA] = s;
-        S[S_BETA] = s / S[S_GAMMA_OLD];
-        if (!isfinite(S[S_BETA])) S[S_DONE] = 3;
+        S[S_BETA] = beta;
+        if (!isfinite(beta)) done = 3;
         break;
-    case FIN_MEAN: S[S_MEAN] = s / s2; break;
+    }
     case FIN_RHS2:
         // |b|^2 turns the relative threshold tol^2 into tol^2 |b|^2; a zero b is solved by
         // x = 0, a non-finite one stops the solve
         S[S_TMP] = s;
         S[S_RHS2] = s;
-        if (!isfinite(s)) S[S_DONE] = 3;
-        else if (s == 0.0) S[S_DONE] = 1;
-        else S[S_THR2] = fmax(S[S_THR2] * s, 2.2250738585072014e-308);
-        break;
-    case FIN_BETA_FLEX:
-        // flexible CG (Polak-Ribiere): beta = z.(r - r_old) / gamma_old = -alpha z.Ap / gamma_old
-        S[S_GAMMA_OLD] = S[S_GAMMA];
-        S[S_GAMMA] = s;
-        S[S_BETA] = -S[S_ALPHA] * s2 / S[S_GAMMA_OLD];
-        if (!isfinite(S[S_BETA])) S[S_DONE] = 3;
+        if (!isfinite(s)) done = 3;
+        else if (s == 0.0) done = 1;
+        else S[S_THR2] = fmax(v[S_THR2] * s, 2.2250738585072014e-308);
         break;
     }
+    S[S_DONE] = done;
+    return done;
 }
 
 // FIN_RR with sig (host-mapped coherent memory): one 64-bit word, the count of FIN_RR launches
@@ -2529,33 +2538,34 @@ __global__ __launch_bounds__(1024) void finish(const double* __restrict__ partia
 {
     __shared__ double red[16];
     __shared__ double red2[16];
-    // the stop flag is read first and tested only before the writes, so that its load
-    // overlaps the partials' (a stopped solve's partials are stale but in bounds)
-    const bool skip = kind != FIN_SUM && kind != FIN_MEAN && S[S_DONE] != 0.0;
+    __shared__ double was[S_COUNT];
+    // the scalars are loaded with the partials and the stop flag tested only before the writes (a
+    // stopped solve's partials are stale but in bounds)
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    if (w == 15 && lane < S_COUNT) was[lane] = S[lane];
     // each thread adds its strided partials in index order
     double v = 0, v2 = 0;
-    if (partial2) finish_terms<16, true>(partial, partial2, n, v, v2);
-    else finish_terms<40, false>(partial, nullptr, n, v, v2);
-    for (int o = 32; o > 0; o >>= 1) {
-        v += __shfl_xor(v, o, 64);
-        v2 += __shfl_xor(v2, o, 64);
+    if (partial2) finish_terms<true>(partial, partial2, n, v, v2);
+    else finish_terms<false>(partial, nullptr, n, v, v2);
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    if (lane == 0) red[w] = v;
+    if (partial2) {
+        for (int o = 32; o > 0; o >>= 1) v2 += __shfl_xor(v2, o, 64);
+        if (lane == 0) red2[w] = v2;
     }
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    if (lane == 0) { red[w] = v; red2[w] = v2; }
     __syncthreads();
     if (threadIdx.x != 0) return;
+    double done = was[S_DONE];
+    if (kind == FIN_SUM || kind == FIN_MEAN || done == 0.0) done = finish_apply(S, was, kind, red, red2);
     if (kind == FIN_RR) {
-        // the stopping test (skipped once the solve has stopped) and its outcome
-        S[S_POLL] += 1;
-        if (!skip) finish_apply(S, kind, red, red2);
+        // the outcome of the stopping test (skipped once the solve has stopped)
+        const double poll = was[S_POLL] + 1;
+        S[S_POLL] = poll;
         if (sig) {
-            const unsigned long long word = (static_cast<unsigned long long>(S[S_POLL]) << 3) |
-                                            static_cast<unsigned long long>(S[S_DONE]);
+            const unsigned long long word = (static_cast<unsigned long long>(poll) << 3) | static_cast<unsigned long long>(done);
             __hip_atomic_store(sig, word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         }
-        return;
     }
-    if (!skip) finish_apply(S, kind, red, red2);
 }
 
 // level-0 FP64 dense solve: x = A0^-1 b on the level's INTERIOR cells.
