@@ -463,7 +463,9 @@ cmg_status cmg_bench_kernel(cmg_solver* s, int kernel, int reps, double* avg_ms,
  * finest-level sweep from x = 0 into the x/r update, sum r.z over each level's
  * LEAF tiles in that level's last post-sweep, which regroups the FP64 partial
  * sums of r.z, do a coarse level's FAS save in its first pre-sweep and the FAS
- * prolongation to the next finer level in its last post-sweep); bit 5 set keeps
+ * prolongation to the next finer level in its last post-sweep; and by default
+ * cycles run levels 0 and 1, and each half of a visit to a complete level, in
+ * one launch, the geometric solvers' levels included); bit 5 set keeps
  * the prolongation into the finest level out of the finest post-sweeps (by
  * default a PCG solve's finest post-sweeps compute it on the fly; the cycle's
  * output on GHOST tiles of the finest level, which PCG never reads, then keeps 0);
