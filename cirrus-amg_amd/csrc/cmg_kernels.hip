@@ -99,13 +99,16 @@ __device__ __forceinline__ float derived_diag(const Lds<T, LQ>& s, int v, const 
 // thread owns CPT = 512/NT cells, v = own_cell<NT>(c) = CPT*tid + c (consecutive
 // along k) for the one-tile-per-workgroup kernels (load_tile), v = tid + c*NT
 // (CPT x-planes apart) for the persistent pipelined forms (issue / stage_lds).
-template <typename T, int NT>
+// LATE: load_tile leaves the derived diagonals to cell_lap, which sets d cell by cell
+template <typename T, int NT, bool LATE = false>
 struct Own {
     static constexpr int CPT = 512 / NT;
     T x[CPT];          // x masked to INTERIOR cells
     float c[CPT][3];   // negative-face coefficients
     float d[CPT];      // diagonal
     uint8_t ct[CPT];   // cell type
+    bool derive;       // LATE: the tile's diagonals are derived
+    bool open[3];      // LATE: the tile has a neighbour across its + face of each axis
 };
 
 // a pointer argument as a workgroup-uniform value (kept in SGPRs, selectable
@@ -177,9 +180,9 @@ struct Pull {
 };
 // Q 2: W and L are the coded form's cell words and tables (Coef::w, Coef::lut); the LDS
 // may be a form-2 one for a form-0 load (a kernel that takes either form per tile).
-template <bool FRESH, typename T, int NT, int Q = 0, typename Extra = NoExtraLoads, typename PullT = Pull<0>, int LQ>
+template <bool FRESH, typename T, int NT, int Q = 0, typename Extra = NoExtraLoads, typename PullT = Pull<0>, int LQ, bool LATE>
 __device__ __forceinline__ void load_tile(const TopoView& tp, const TileRec& r, float h, const T* __restrict__ X,
-                                          const T* __restrict__ G, const float* const* C, Lds<T, LQ>& s, Own<T, NT>& o,
+                                          const T* __restrict__ G, const float* const* C, Lds<T, LQ>& s, Own<T, NT, LATE>& o,
                                           const uint16_t* const* Qc = nullptr, const Extra& extra = Extra{},
                                           const PullT& pull = PullT{nullptr, 0.0f}, const uint32_t* __restrict__ W = nullptr,
                                           const float* __restrict__ L = nullptr, const uint32_t* __restrict__ ZW = nullptr)
@@ -510,7 +513,12 @@ __device__ __forceinline__ void load_tile(const TopoView& tp, const TileRec& r, 
         }
     }
     __syncthreads();
-    if constexpr (Q != 1) {
+    if constexpr (LATE) {
+        o.derive = dv;
+        o.open[0] = ha.w >= 0;
+        o.open[1] = hb.x >= 0;
+        o.open[2] = hb.y >= 0;
+    } else if constexpr (Q != 1) {
         if (dv) {
 #pragma unroll
             for (int c = 0; c < CPT; ++c) {
@@ -520,6 +528,49 @@ __device__ __forceinline__ void load_tile(const TopoView& tp, const TileRec& r, 
             }
         }
     }
+}
+
+// neg_lap of a thread's cell c, with the diagonal that load_tile left to it (derived_diag's sum):
+// the + face coefficients are read once for both, and what the thread's next and last cell
+// along k hold comes from registers: 24 instead of 45 LDS reads for a thread's four cells on a
+// coded LEAF tile (a + face's code and its table entry count as two).  The 1024^3 torus: finest r.z
+// sweep 61.1 -> 57.9 us, operator 87.3 -> 83.0, restriction 49.1 -> 47.9, a solve 10.04 -> 9.88 ms;
+// the 256^3 sphere 3.02 -> 2.98.  (Scalar halo addresses beside it, a quarter fewer vector
+// instructions: 10.01 and 3.05 ms.)
+template <int NT, int LQ>
+__device__ __forceinline__ float cell_lap(const Lds<float, LQ>& s, Own<float, NT, true>& o, int c, int tid, float h)
+{
+    constexpr int CPT = 512 / NT;
+    const int v = own_cell<NT>(c, tid);
+    if (o.derive ? !(o.ct[c] & INTERIOR) : o.d[c] == 0) {
+        if (o.derive) o.d[c] = 0.0f;
+        return 0.0f;
+    }
+    const int i = v >> 6, j = (v >> 3) & 7, k = v & 7;
+    const bool next = c + 1 < CPT, last = c > 0;
+    const float cp0 = staged_coef(s, 0, i < 7 ? v + 64 : 512 + (j * 8 + k), h);
+    const float cp1 = staged_coef(s, 1, j < 7 ? v + 8 : 512 + (i * 8 + k), h);
+    const float cp2 = next ? o.c[next ? c + 1 : c][2] : staged_coef(s, 2, k < 7 ? v + 1 : 512 + (i * 8 + j), h);
+    float d = o.d[c];
+    if (o.derive) {
+        d = 0.0f;
+        d = d - o.c[c][0];
+        d = d - (i == 7 && !o.open[0] ? -h : cp0);
+        d = d - o.c[c][1];
+        d = d - (j == 7 && !o.open[1] ? -h : cp1);
+        d = d - o.c[c][2];
+        d = d - (k == 7 && !o.open[2] ? -h : cp2);
+        o.d[c] = d;
+        if (d == 0) return 0.0f;
+    }
+    float r = o.x[c] * d;
+    r = fmaf(o.c[c][0], s.x[SX(i - 1, j, k)], r);
+    r = fmaf(cp0, s.x[SX(i + 1, j, k)], r);
+    r = fmaf(o.c[c][1], s.x[SX(i, j - 1, k)], r);
+    r = fmaf(cp1, s.x[SX(i, j + 1, k)], r);
+    r = fmaf(o.c[c][2], last ? o.x[last ? c - 1 : c] : s.x[SX(i, j, k - 1)], r);
+    r = fmaf(cp2, next ? o.x[next ? c + 1 : c] : s.x[SX(i, j, k + 1)], r);
+    return r;
 }
 
 // AMGLaplacianTileData::negativeLap (src/AMGSolver.cu:345-382) for cell v
@@ -1321,12 +1372,13 @@ __global__ __launch_bounds__(NT) void apply_leaf(TopoView tp, const int4* __rest
         if (DOT && t == -1 && threadIdx.x == 0) partial[blockIdx.x] = 0;
         return;
     }
-    Own<float, NT> o;
+    Own<float, NT, true> o;
+    const float h = rec_h(tp, r);
     if (K && (((C.coded & ~C.wide) >> r.level) & 1u))
-        load_tile<true, float, NT, K ? 3 : 0>(tp, r, rec_h(tp, r), X, X, C.c, s, o, nullptr, NoExtraLoads{},
+        load_tile<true, float, NT, K ? 3 : 0>(tp, r, h, X, X, C.c, s, o, nullptr, NoExtraLoads{},
                                              Pull<0>{nullptr, 0.0f}, C.w, C.lut, C.zw);
     else
-        load_tile<true, float, NT, 0>(tp, r, rec_h(tp, r), X, X, C.c, s, o);
+        load_tile<true, float, NT, 0>(tp, r, h, X, X, C.c, s, o);
     constexpr int CPT = 512 / NT;
     const size_t v0 = size_t(t) * 512 + size_t(CPT) * threadIdx.x;
     float xr[CPT], y[CPT];
@@ -1334,8 +1386,8 @@ __global__ __launch_bounds__(NT) void apply_leaf(TopoView tp, const int4* __rest
     double acc = 0;
 #pragma unroll
     for (int c = 0; c < CPT; ++c) {
-        const int v = own_cell<NT>(c);
-        y[c] = o.ct[c] == INTERIOR ? neg_lap(s, v, o.x[c], o.c[c], o.d[c]) : 0.0f;
+        const float ax = cell_lap(s, o, c, threadIdx.x, h);
+        y[c] = o.ct[c] == INTERIOR ? ax : 0.0f;
         if (DOT) acc += double(xr[c]) * double(y[c]);
     }
     vstore<CPT>(Y + v0, y);
@@ -1454,7 +1506,7 @@ __device__ __forceinline__ double jacobi_tile(const TopoView& tp, const TileRec&
 {
     static_assert(!(SAVE && PUSH), "the FAS save rides on a first sweep, the prolongation on a last one");
     const int t = r.t, tid = r.tid;
-    Own<float, NT> o;
+    Own<float, NT, true> o;
     constexpr int CPT = 512 / NT;
     const size_t v0 = size_t(t) * 512 + size_t(CPT) * tid;
     float b[CPT], xo[CPT];
@@ -1500,7 +1552,7 @@ __device__ __forceinline__ double jacobi_tile(const TopoView& tp, const TileRec&
 #pragma unroll
     for (int c = 0; c < CPT; ++c) {
         const int v = own_cell<NT>(c, tid);
-        const float ax = neg_lap(s, v, o.x[c], o.c[c], o.d[c], h);
+        const float ax = cell_lap(s, o, c, tid, h);
         if (save) {
             const size_t idx = size_t(t) * 512 + v;
             if (o.ct[c] & INTERIOR) {
@@ -1587,14 +1639,14 @@ __device__ __forceinline__ void residual_restrict_tile(const TopoView& tp, const
                                                        float* __restrict__ B, float Rr, bool act)
 {
     const int t = r.t, tid = r.tid;
-    Own<float, NT> o;
+    Own<float, NT, true> o;
     constexpr int CPT = 512 / NT;
     float b[CPT], rv[CPT];
     vload<CPT>(B + size_t(t) * 512 + size_t(CPT) * tid, b);
     const float h = rec_h(tp, r);
     load_tile<false, float, NT, Q>(tp, r, h, X, X, C.c, s, o, C.q, NoExtraLoads{}, Pull<0>{nullptr, 0.0f}, C.w, C.lut, C.zw);
 #pragma unroll
-    for (int c = 0; c < CPT; ++c) rv[c] = b[c] - neg_lap(s, own_cell<NT>(c, tid), o.x[c], o.c[c], o.d[c], h);
+    for (int c = 0; c < CPT; ++c) rv[c] = b[c] - cell_lap(s, o, c, tid, h);
     vstore<CPT>(&res[CPT * tid], rv);
     __syncthreads();
     const int v = tid;
