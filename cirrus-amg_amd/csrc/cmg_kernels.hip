@@ -532,7 +532,7 @@ __device__ __forceinline__ void load_tile(const TopoView& tp, const TileRec& r, 
 
 // neg_lap of a thread's cell c, with the diagonal that load_tile left to it (derived_diag's sum):
 // the + face coefficients are read once for both, and what the thread's next and last cell
-// along k hold comes from registers: 24 instead of 45 LDS reads for a thread's four cells on a
+// along k hold comes from registers: 36 instead of 72 LDS reads for a thread's four cells on a
 // coded LEAF tile (a + face's code and its table entry count as two).  The 1024^3 torus: finest r.z
 // sweep 61.1 -> 57.9 us, operator 87.3 -> 83.0, restriction 49.1 -> 47.9, a solve 10.04 -> 9.88 ms;
 // the 256^3 sphere 3.02 -> 2.98.  (Scalar halo addresses beside it, a quarter fewer vector
