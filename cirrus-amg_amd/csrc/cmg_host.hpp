@@ -121,6 +121,11 @@ private:
     std::array<ZeroArray<int32_t>, kMaxLevels> slot_tile_;      // slot -> tile index + 1, 0 for none
 };
 
+// the tiles of a level that fills the cube of the level-0 tile `root` with its 8^level LEAF or NONLEAF
+// tiles and has no other tile, by their place (x * 2^level + y) * 2^level + z in that cube, wherever
+// the root lies; empty for any other level
+std::vector<int32_t> complete_level(const Topology& topo, int root, int level);
+
 // analytic SDFs shared by targets and assembly (float, no contraction)
 float sdf_eval(int kind, const float* prm, float x, float y, float z);
 std::function<int(int, const Coord&)> make_target(const Topology& topo, const cmg_target& t);

@@ -394,24 +394,29 @@ void dev_upload(DevGrid& d, const Topology& topo)
             d.bottom_ok = kids;
         }
     }
-    for (int l = 1; d.root_alone && l < topo.num_levels() && l < kMaxLevels; ++l) {
-        const size_t n = size_t(1) << (3 * l);
-        if (n > kDenseTiles || sub[l].size() != n || pr[l].size() != n) break;
-        const int e = 1 << l;   // tiles along an edge
-        std::vector<int32_t> at(n);
-        auto place = [&](int x, int y, int z) { return (size_t(x) * e + y) * e + z; };
-        for (int t : sub[l]) at[place(topo.t_coord[t][0], topo.t_coord[t][1], topo.t_coord[t][2])] = t;
+    for (int l = 1; d.root_alone && l < topo.num_levels() && l < kMaxLevels && (size_t(1) << (3 * l)) <= kDenseTiles; ++l) {
+        const int root = sub[0][0], e = 1 << l;   // tiles along an edge
+        const std::vector<int32_t> at = complete_level(topo, root, l);
+        if (at.empty()) break;
         const std::vector<int32_t>& order = d.subtree[l].order;
         std::vector<int32_t> tab(order.size() * kDenseWords, -1);
-        bool whole = order.size() == n;   // no padding entries
+        bool whole = order.size() == at.size();   // no padding entries
         for (size_t i = 0; whole && i < order.size(); ++i) {
             const int t = order[i];
             int32_t* w = &tab[i * kDenseWords];
             int32_t nonleaf = 0;
             for (int o = 0; o < 27; ++o) {
-                const int x = topo.t_coord[t][0] + o / 9 - 1, y = topo.t_coord[t][1] + o / 3 % 3 - 1, z = topo.t_coord[t][2] + o % 3 - 1;
-                if (x < 0 || x >= e || y < 0 || y >= e || z < 0 || z >= e) continue;
-                w[o] = at[place(x, y, z)];
+                const int step[3] = {o / 9 - 1, o / 3 % 3 - 1, o % 3 - 1};
+                bool inside = true;
+                size_t place = 0;
+                for (int a = 0; a < 3; ++a) {
+                    // relative to the root's cube, which may lie anywhere
+                    const int c = int(topo.t_coord[t][a] - int64_t(topo.t_coord[root][a]) * e) + step[a];
+                    inside = inside && c >= 0 && c < e;
+                    place = place * size_t(e) + size_t(c);
+                }
+                if (!inside) continue;
+                w[o] = at[place];
                 w[27 + o] = topo.parent[w[o]];
                 if (topo.t_type[w[o]] & NONLEAF) nonleaf |= 1 << o;
             }

@@ -218,6 +218,26 @@ void Topology::finalize()
     finalized_ = true;
 }
 
+std::vector<int32_t> complete_level(const Topology& topo, int root, int level)
+{
+    const int lo = topo.level_start[level], hi = topo.level_start[level + 1];
+    const size_t n = size_t(1) << (3 * level);
+    if (size_t(hi - lo) != n) return {};
+    const int64_t e = int64_t(1) << level;   // tiles along an edge
+    std::vector<int32_t> at(n);
+    for (int t = lo; t < hi; ++t) {
+        if (!(topo.t_type[t] & (LEAF | NONLEAF))) return {};
+        size_t place = 0;
+        for (int a = 0; a < 3; ++a) {
+            const int64_t c = topo.t_coord[t][a] - topo.t_coord[root][a] * e;
+            if (c < 0 || c >= e) return {};
+            place = place * size_t(e) + size_t(c);
+        }
+        at[place] = t;   // (a level's coordinates are distinct: n of them inside the cube fill it)
+    }
+    return at;
+}
+
 // ---------------------------------------------------------------- targets ---
 
 float sdf_eval(int kind, const float* p, float x, float y, float z)
