@@ -12,7 +12,7 @@
 //     r.z partials and the prolongation to the level above (fas_prolong_v, gs_color or
 //     jacobi); x goes from T to X, the saved right-hand side to B
 // Every value is computed with the operations of the kernels named, so the results are the
-// same bits.
+// same bits, but where a quotient lies halfway between two subnormal numbers (quotient()).
 //
 // What bounds the kernels they replace on such levels is the latency of a launch, 4 to 5 us
 // whatever its work: a red-black visit of two sweeps each way took eleven launches, a Jacobi

@@ -273,7 +273,8 @@ __device__ __forceinline__ float geo_lap6(float h, float K, uint32_t open, float
 // computes the halo's cells again, so no pass waits for the neighbours.  POST false: the
 // red-black iterations from x = 0 (x into T), the residual and its restriction into B below;
 // true: the prolongation (prolong_add_v) onto T, the iterations from black, x into X.  The
-// operations are those of geo_gs, geo_restrict and prolong_add_v.  At most two iterations.
+// operations are those of geo_gs, geo_restrict and prolong_add_v, with quotient() in the place
+// of the division.  At most two iterations.
 // Bound by launch latency before (ten launches of about 4 us a visit) and by the issue of the
 // halo's work now: MI355X, GMG, 11.3 + 10.7 us a visit to 512 tiles, 7.9 + 7.0 us to 64.
 constexpr int kGeoRow = 21, kGeoPlane = 18 * kGeoRow;   // x in LDS, see cmg_dense.hip

@@ -1882,7 +1882,8 @@ __device__ __forceinline__ TileRec rec_tile_at(const int4* __restrict__ r, int t
 // right-hand side stay in LDS too, and its 512 cells are two a thread, one of each colour,
 // on the first 256 threads.  Every step does the arithmetic of the per-pass kernel it
 // replaces (gs_color, jacobi, residual_restrict, fas_save, coarsest_tile, fas_prolong_v,
-// jacobi's r.z partial), so the results are bit-identical.
+// jacobi's r.z partial), so the results are bit-identical, but where a quotient lies halfway
+// between two subnormal numbers (quotient()).
 // PHASE 1: level 1's FAS save, pre-smoothing, residual + restriction, the root's FAS save;
 // PHASE 2: the prolongation to level 1, its post-smoothing and the prolongation into level
 // 2; PHASE 3: both with the coarsest iterations (mu times) in between, `visits` times in a row.

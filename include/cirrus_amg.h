@@ -482,7 +482,10 @@ cmg_status cmg_bench_kernel(cmg_solver* s, int kernel, int reps, double* avg_ms,
  * bits 0-2 read the FP32 channels).
  * stencil_threads: 128, 256 or 512 threads per tile, or 0 for the library's
  * defaults (CMG_STENCIL_THREADS when set).  Stencil results are
- * bit-identical across forms; PCG scalars differ only by the grouping of FP64
+ * bit-identical across forms, but for one rounding: the launches that bit 4 turns
+ * off multiply by FP64 reciprocals, and a quotient b / d exactly halfway between two
+ * subnormal numbers (d a multiple of 2) may there become either of them, 2^-149
+ * apart.  PCG scalars differ only by the grouping of FP64
  * partial sums.  Default: mask 0, 256 threads (the Jacobi sweep on FP16 coefficient
  * copies: 128 until a thread count is set here or by CMG_STENCIL_THREADS).  No reference counterpart (the reference
  * kernels have one fixed form, src/AMGSolver.cu:589-632, 838-964).  Returns
