@@ -310,11 +310,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void d
     } else {
         for (int p = 0; p < passes; ++p) {
             const bool go = dep <= deep - p;
+            const bool zero = !POST && a.zero && p == 0;   // w b / d, also where a coefficient is not finite
             float xo[8];
             if (go) {
 #pragma unroll
                 for (int c = 0; c < 8; ++c) {
-                    const float delta = interior(c) ? quotient(b[c] - lap(c), rd[c]) : 0.0f;
+                    const float ax = lap(c);
+                    const float delta = interior(c) ? quotient(b[c] - (zero ? 0.0f : ax), rd[c]) : 0.0f;
                     xo[c] = x[c] + a.w * delta;
                 }
             }

@@ -1,6 +1,6 @@
 """The quotients of the fused visits (a product with an FP64 reciprocal) against the per-pass kernels' division, bit for
 bit, through cycles on an operator without face coefficients, where a pass is b / d alone: all exponents, quotients next
-to midpoints, subnormal diagonals, right-hand sides and quotients."""
+to midpoints, subnormal diagonals, right-hand sides and quotients, zeros, infinities and NaN."""
 import numpy as np
 import pytest
 
@@ -26,7 +26,8 @@ def _pairs(kind, n, rng):
         bits = np.where((bits >> 23) & 0xff == 0xff, bits ^ np.uint32(1 << 23), bits)   # finite
         bits = (bits & np.uint32(0xff800000)) | edge[rng.integers(0, 7, (2, n))]
         return bits[0].view(np.float32), bits[1].view(np.float32)
-    raise ValueError(kind)
+    special = np.array([0, -0.0, np.inf, -np.inf, np.nan, 2.0**-149, 2.0**-126, 3.4e38, 1, -1], np.float32)
+    return rng.choice(special, n), rng.choice(special, n)
 
 
 def _no_ties(n, d):
@@ -39,7 +40,7 @@ def _no_ties(n, d):
 
 @pytest.mark.parametrize("level", [2, 1, 0])
 @pytest.mark.parametrize("smoother", [0, 1])
-@pytest.mark.parametrize("kind", ["subnormal", "midpoints", "extremes"])
+@pytest.mark.parametrize("kind", ["subnormal", "midpoints", "extremes", "special"])
 def test_quotients_of_fused_visits(kind, smoother, level):
     print("\nquotient", kind, smoother, level, flush=True)
     _, g = H.build_pair("uniform2")
