@@ -250,7 +250,8 @@ void launch_coarsest_iterate(const DevGrid& d, float* X, Coef C, const float* B,
                              double omega, float w, const double* S, hipStream_t st);
 // the inverse of a symmetric n x n matrix (n <= 4096: `shift` everywhere plus the given entries,
 // row << 16 | column, no place twice) into inv (cmg_inverse.hip); false when a pivot of the
-// elimination is not positive or nearly 0 (inv is then not an inverse).  Synchronises the stream.
+// elimination is not positive or nearly 0, or where the device has no room for its two work matrices
+// (inv is then not an inverse).  Synchronises the stream.
 bool device_inverse(int n, double shift, const std::vector<uint32_t>& rc, const std::vector<double>& v, double* inv,
                     hipStream_t st);
 void launch_coarse_direct(const double* inv, const int32_t* cells, int n, const int32_t* zero_cells, int nz, float* X,

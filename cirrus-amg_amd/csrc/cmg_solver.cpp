@@ -902,7 +902,7 @@ void build_direct(cmg_solver* s, bool pure_neumann)
     double* const dinv = dmalloc<double>(size_t(n) * n);
     try {
         // on the device when the matrix is symmetric and its elimination meets positive pivots only
-        // (every operator assembled here); else with partial pivoting on the host
+        // (every operator assembled here) and has room there; else with partial pivoting on the host
         if (!(n > 0 && symmetric(rows) && inverse_on_device(n, shift, rows, dinv, d.stream))) {
             const std::vector<double> inv = pivoted_inverse(n, shift, rows);
             if (n) HIPCHK(hipMemcpy(dinv, inv.data(), inv.size() * sizeof(double), hipMemcpyHostToDevice));

@@ -1,5 +1,8 @@
 """The FP64 direct solve of level 0: its inverse is made on the device for symmetric positive definite systems (sizes off
 the elimination's blocks among them) and on the host otherwise; both solve the level-0 system."""
+import os
+import subprocess
+
 import numpy as np
 import pytest
 
@@ -89,3 +92,12 @@ def test_pure_neumann_solve():
     o = P.default_opts(cycle=P.CYCLE_FAS_V, smoother=P.SMOOTH_JACOBI, omega=2.0 / 3.0, coarsest_direct=1)
     it, rel = P.AMGSolver(gp, H.C0, H.R_MATRIX, 1.0, 1.0).solve(relative_tolerance=1e-6, is_pure_neumann=True, opts=o)
     assert rel < 1e-6 and it < 40
+
+
+def test_no_room_for_the_device_inverse():
+    """the workspace's allocation refused (from the host, by the test program's own hipMalloc): the same solution"""
+    cpp = os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpp")
+    subprocess.run(["make", "-s", "-C", cpp, "_build/test_inverse_fallback"], check=True)
+    print("\ninverse fallback", flush=True)
+    r = subprocess.run([os.path.join(cpp, "_build", "test_inverse_fallback")], capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0 and "inverse fallback OK" in r.stdout, r.stdout + r.stderr
