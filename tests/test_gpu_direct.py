@@ -1,5 +1,6 @@
 """The FP64 direct solve of level 0: its inverse is made on the device for symmetric positive definite systems (sizes off
-the elimination's blocks among them) and on the host otherwise; both solve the level-0 system."""
+the elimination's blocks and the largest one among them) and on the host otherwise; both solve the level-0 system.  The
+unpivoted elimination inverts an unsymmetric system with positive pivots as well, so no case tells which of the two ran."""
 import os
 import subprocess
 
@@ -13,13 +14,14 @@ pytestmark = pytest.mark.gpu
 
 
 def _grid(case):
-    """a single-level grid of one tile (so that a cycle is the direct solve), its types and operator"""
+    """a single-level grid of one tile, or of eight (so that a cycle is the direct solve), its types and operator"""
     g = P.HADeviceGrid(log2_hash=(4,))
-    g.setTileHost(0, (0, 0, 0), P.LEAF)
+    for o in range(8 if case == "largest" else 1):
+        g.setTileHost(0, (o & 1, o >> 1 & 1, o >> 2 & 1), P.LEAF)
     g.rebuild()
     g.finalize()
     rng = np.random.default_rng(5)
-    types = np.full((1, 512), P.INTERIOR, np.uint8)
+    types = np.full((g.N, 512), P.INTERIOR, np.uint8)
     if case == "ragged":       # 512 - 75 unknowns: not a multiple of 32
         types[0, rng.choice(512, 75, replace=False)] = P.DIRICHLET
     if case == "few":          # a few unknowns only
@@ -31,49 +33,59 @@ def _grid(case):
 
 
 def _matrix(g):
-    """the level-0 system from the grid's types and coefficients"""
-    C = [g.channel(H.C0 + a)[0].astype(np.float64) for a in range(4)]
-    inside = g.cell_types()[0] == P.INTERIOR
-    cells = np.where(inside)[0]
+    """the level-0 system from the grid's types and coefficients (a cell without diagonal has an empty row)"""
+    C = [g.channel(H.C0 + a).astype(np.float64) for a in range(4)]
+    co = g.tiles()[1]
+    v = np.arange(512)
+    at = (co[:, None] * 8 + np.stack([v >> 6, (v >> 3) & 7, v & 7], 1)).reshape(-1, 3)
+    cells = np.where(g.cell_types().ravel() == P.INTERIOR)[0]
+    place = {tuple(at[c]): c for c in range(len(at))}
     uid = {c: i for i, c in enumerate(cells)}
     A = np.zeros((len(cells), len(cells)))
     for i, c in enumerate(cells):
-        l = [c >> 6, (c >> 3) & 7, c & 7]
-        A[i, i] = C[3][c]
-        for a, step in enumerate((64, 8, 1)):
-            if l[a] > 0 and c - step in uid:
-                A[i, uid[c - step]] += C[a][c]
-            if l[a] < 7 and c + step in uid:
-                A[i, uid[c + step]] += C[a][c + step]
+        A[i, i] = C[3].ravel()[c]
+        if A[i, i] == 0:
+            continue
+        for a in range(3):
+            for side in (-1, 1):
+                n = list(at[c])
+                n[a] += side
+                n = place.get(tuple(n))
+                if n in uid:
+                    A[i, uid[n]] += C[a].ravel()[c if side < 0 else n]
     return cells, A
 
 
-@pytest.mark.parametrize("case", ["full", "ragged", "few", "unsymmetric", "indefinite"])
+@pytest.mark.parametrize("case", ["full", "ragged", "few", "largest", "indefinite", "singular", "unsymmetric"])
 def test_level0_direct_solve(case):
+    print("\ndirect", case, flush=True)
     g = _grid(case)
-    if case in ("unsymmetric", "indefinite"):
-        # a diagonal of its own for some cells: still diagonally dominant, no longer definite when negative;
-        # a face coefficient seen from one side only cannot be made here, so the unsymmetric form drops a
-        # diagonal, which leaves that cell's row empty and the system singular
+    if case in ("indefinite", "singular", "unsymmetric"):
+        # a diagonal of its own for one cell: not definite where it is negative; 0 leaves the cell's row empty
+        # and the system singular, and with the shift of a pure Neumann system regular and unsymmetric
         d = g.channel(H.C0 + 3)
-        d[0, 77] = 0.0 if case == "unsymmetric" else -8.0
+        d[0, 77] = -8.0 if case == "indefinite" else 0.0
         g.set_channel(H.C0 + 3, d)
     cells, A = _matrix(g)
-    b = H.random_fill(1, 9)
+    b = H.random_fill(g.N, 9)
     g.set_channel(1, b)
-    o = P.default_opts(cycle=P.CYCLE_FAS_V, smoother=P.SMOOTH_JACOBI, coarsest_direct=1)
-    s = P.AMGSolver(g, H.C0, H.R_MATRIX, 1.0, 1.0)
+    o = P.default_opts(cycle=P.CYCLE_FAS_V, smoother=P.SMOOTH_JACOBI, coarsest_direct=1,
+                       is_pure_neumann=int(case == "unsymmetric"))
     if case == "unsymmetric":
+        assert not np.array_equal(A, A.T)
+        A = A + np.trace(A) / len(cells) ** 2
+    s = P.AMGSolver(g, H.C0, H.R_MATRIX, 1.0, 1.0)
+    if case == "singular":
         with pytest.raises(P.CmgError) as e:
             s.cycle(o, 4, 1, 3)
         assert "singular" in str(e.value)
         return
     s.cycle(o, 4, 1, 3)
-    x = np.linalg.solve(A, b[0, cells].astype(np.float64))
-    z = g.channel(4)[0]
+    x = np.linalg.solve(A, b.ravel()[cells].astype(np.float64))
+    z = g.channel(4).ravel()
     # the FP32 result of an FP64 solve: half an ulp, and the FP64 error of a condition number below 1e4
     assert np.abs(z[cells] - x).max() <= 2.0**-24 * np.abs(x).max() * 1.01
-    rest = np.setdiff1d(np.arange(512), cells)
+    rest = np.setdiff1d(np.arange(z.size), cells)
     assert not z[rest].any()
 
 
