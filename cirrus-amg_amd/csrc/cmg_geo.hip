@@ -243,7 +243,7 @@ __global__ __launch_bounds__(256) void geo_restrict(TopoView tp, const int4* __r
 }
 
 // Face coefficients and diagonals where every cell of the neighbourhood belongs to the level (no
-// GHOST tile): an open face has geo_coeff's value K, one next to a NEUMANN cell 0, so a cell's
+// GHOST tile): an open face has geo_open_coeff's value K, one next to a NEUMANN cell 0, so a cell's
 // coefficients are six bits and its diagonal one of seven values.
 template <int MODE>
 __device__ __forceinline__ float geo_face(float h)

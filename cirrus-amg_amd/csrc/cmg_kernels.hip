@@ -1765,7 +1765,7 @@ __global__ __launch_bounds__(NT) void gs_color(TopoView tp, const int4* __restri
 template <int NT, int Q = 0>
 __device__ __forceinline__ void coarsest_tile(const TopoView& tp, const TileRec& r, Lds<float, Q>& s, float* __restrict__ X,
                                               const Coef& C, const float* __restrict__ B, int rbgs, int iters, int iters2,
-                                              int order, double omega, float w, bool act)
+                                              int order, double omega, float w)
 {
     const int t = r.t, tid = r.tid;
     Own<float, NT> o;
@@ -1799,7 +1799,7 @@ __device__ __forceinline__ void coarsest_tile(const TopoView& tp, const TileRec&
         __syncthreads();
     }
     // every cell was written by a pass (rbgs: both colours ran at least once)
-    if (act) vstore<CPT>(X + v0, xn);
+    vstore<CPT>(X + v0, xn);
 }
 
 template <int NT, int Q = 0>
@@ -1811,7 +1811,7 @@ __global__ __launch_bounds__(NT) void coarsest_iterate(TopoView tp, const int4* 
     __shared__ Lds<float, Q> s;
     const TileRec r = rec_tile<false>(rec, S);
     if (r.t < 0) return;   // no tile, or the solve has stopped
-    coarsest_tile<NT, Q>(tp, r, s, X, C, B, rbgs, iters, iters2, order, omega, w, true);
+    coarsest_tile<NT, Q>(tp, r, s, X, C, B, rbgs, iters, iters2, order, omega, w);
 }
 
 // ------------------------------------------------------------- transfers ----
@@ -1819,7 +1819,7 @@ __global__ __launch_bounds__(NT) void coarsest_iterate(TopoView tp, const int4* 
 template <int NT, int Q = 0>
 __device__ __forceinline__ void fas_save_tile(const TopoView& tp, const TileRec& r, Lds<float, Q>& s,
                                               const float* __restrict__ X, const Coef& C, float* __restrict__ B,
-                                              float* __restrict__ X0, bool act)
+                                              float* __restrict__ X0)
 {
     const int t = r.t, tid = r.tid;
     Own<float, NT> o;
@@ -1829,7 +1829,6 @@ __device__ __forceinline__ void fas_save_tile(const TopoView& tp, const TileRec&
     vload<CPT>(B + v0, bv);
     const float h = rec_h(tp, r);
     load_tile<false, float, NT, Q>(tp, r, h, X, X, C.c, s, o, C.q, NoExtraLoads{}, Pull<0>{nullptr, 0.0f}, C.w, C.lut, C.zw);
-    if (!act) return;
 #pragma unroll
     for (int c = 0; c < CPT; ++c) {
         if (o.ct[c] & INTERIOR) {
@@ -1850,26 +1849,7 @@ __global__ __launch_bounds__(NT) void fas_save(TopoView tp, const int4* __restri
     __shared__ Lds<float, Q> s;
     const TileRec r = rec_tile<false>(rec, S);
     if (r.t < 0) return;   // no tile, or the solve has stopped
-    fas_save_tile<NT, Q>(tp, r, s, X, C, B, X0, true);
-}
-
-// a record read at a given address (not from the launch list position), thread index tid
-__device__ __forceinline__ TileRec rec_tile_at(const int4* __restrict__ r, int tid)
-{
-    TileRec x;
-    const int4 r0 = r[0];
-    x.t = r0.x;
-    x.level = r0.y;
-    x.meta = r0.z;
-    x.parent = r0.w;
-    x.ha = r[1];
-    x.hb = r[2];
-    x.ga = make_int4(-1, -1, -1, -1);
-    x.gb = make_int4(-1, -1, 0, 0);
-    x.ca = r[5];
-    x.cb = r[6];
-    x.tid = tid;
-    return x;
+    fas_save_tile<NT, Q>(tp, r, s, X, C, B, X0);
 }
 
 // The bottom of a FAS mu-cycle, FASMuCycleStep at level 1 with everything below it

@@ -620,6 +620,7 @@ __global__ __launch_bounds__(256) void adam(float* __restrict__ W, float* __rest
 //                     volume and the padding stay 0)
 //   [80688, 81648)    layer 3's weights, bf16 [5 pairs][2 taps][2 halves of 8 ci][3 planes][8 ci]
 constexpr int IL_A1 = 0, IL_A2 = 44912, IL_X = 77232, IL_W3 = 80688, IL_BYTES = 81648;
+static_assert(2 * IL_BYTES <= 160 * 1024, "two workgroups' LDS on a CU");
 constexpr int IL_HALF = 1343 * 16;   // from a1's lower channels to its upper ones
 __device__ __forceinline__ int a1_place(int i, int j, int k) { return IL_A1 + (133 + (i * 11 + j) * 11 + k) * 16; }
 constexpr int IN_PT = 2;   // input cells per thread (896 = 512 own + 384 halo, 512 threads)
@@ -936,7 +937,7 @@ void launch_net_infer(const DevGrid& d, const LaunchList& l, const float* R, con
         return true;
     }();
     (void)attr;
-    // persistent: two workgroups per CU (68 KB of LDS each)
+    // persistent: two workgroups per CU
     const int grid = std::max(1, std::min(l.n, d.wg_cap / 4));
     k::net_infer<<<grid, 512, k::IL_BYTES, st>>>(view(d), l.d, l.n, R, D, W, Y, S);
 }
