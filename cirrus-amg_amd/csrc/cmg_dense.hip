@@ -400,6 +400,9 @@ static void dense_launch(const DevGrid& d, int n, int form, const k::DenseArgs& 
     }
 }
 
+// four passes are what the 16^3 cells hold (the residual needs one cell more).  Jacobi with three and four sweeps,
+// eight iterations with a V-cycle, a launch a pass against this: uniform 64^3 955 -> 766 us and 997 -> 821 us, the
+// 256^3 sphere 2,408 -> 2,177 and 2,590 -> 2,403 (two sweeps: the figures above)
 bool dense_visit_fits(bool rbgs, int iters) { return iters >= 1 && iters <= (rbgs ? 2 : 4); }
 
 void launch_dense_visit(const DevGrid& d, int level, bool post, float* X, float* T, float* B, float* BN, float* X0, Coef C,

@@ -481,7 +481,9 @@ cmg_status cmg_bench_kernel(cmg_solver* s, int kernel, int reps, double* avg_ms,
  * coefficient channels or the cell types are written; the persistent forms of
  * bits 0-2 read the FP32 channels).
  * stencil_threads: 128, 256 or 512 threads per tile, or 0 for the library's
- * defaults (CMG_STENCIL_THREADS when set).  Stencil results are
+ * defaults (CMG_STENCIL_THREADS when set); the launches that do a whole visit to
+ * levels 0 and 1 or to a complete level have 256 to 1024 threads of their own,
+ * whatever is chosen here (bit 4 turns them off).  Stencil results are
  * bit-identical across forms, but for one rounding: the launches that bit 4 turns
  * off multiply by FP64 reciprocals, and a quotient b / d exactly halfway between two
  * subnormal numbers (d a multiple of 2) may there become either of them, 2^-149

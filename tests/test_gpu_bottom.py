@@ -1,5 +1,6 @@
 """The bottom two levels of a FAS cycle in one workgroup, against the oracle bit for bit, over the sweep counts,
-smoothers and repetitions that change its path; and the quotient it divides with."""
+smoothers and repetitions that change its path; and the formula of the quotient it divides with (the device's own
+reciprocal: test_gpu_quotient.py)."""
 import numpy as np
 import pytest
 
